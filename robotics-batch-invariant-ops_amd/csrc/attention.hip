@@ -43,8 +43,7 @@ __global__ __launch_bounds__(256) void attn_softmax_kernel(AttnSoftmaxArgs a) {
   else if (a.mask_kind == 2)
     ar.mask = reinterpret_cast<const T*>(a.mask) + b * a.mB + h * a.mH + i * a.mI;
   T* row = reinterpret_cast<T*>(a.s) + r * a.ld;
-  const bool v = (reinterpret_cast<uintptr_t>(a.s) % 16 == 0) && ((a.ld * sizeof(T)) % 16 == 0);
-  softmax_row<T, T, kAttn>(row, row, a.lk, v, v, ar);
+  attn_softmax_row<T>(row, a.lk, ar);
 }
 
 struct VarlenSoftmaxArgs {
@@ -82,8 +81,7 @@ __global__ __launch_bounds__(256) void varlen_softmax_kernel(VarlenSoftmaxArgs a
   ar.mask_kind = 0;
   ar.mask_stride = 0;
   T* row = reinterpret_cast<T*>(a.s) + soff + (h * ql + i) * lds;
-  const bool v = (reinterpret_cast<uintptr_t>(row) % 16) == 0;
-  softmax_row<T, T, kAttn>(row, row, kl, v, v, ar);
+  attn_softmax_row<T>(row, kl, ar);
 }
 
 }  // namespace biops

@@ -4,9 +4,12 @@
 // elements is cut into 16-byte chunks of VEC input elements; lane L of the wavefront owning the
 // row takes chunks L, L+64, L+128, ... and adds their elements in increasing column order into
 // one fp32 partial; the 64 partials are then combined by the xor butterfly (offsets 32, 16, 8,
-// 4, 2, 1).  Because fp32 addition is commutative, every lane ends with the same bits, and the
-// tree depends only on C and VEC (the input element size) -- not on the number of rows, the
-// row's position, or whether the row was read once (kept in registers) or several times.
+// 4, 2, 1).  Rows too long for one wavefront's registers go to a workgroup of T threads: thread t
+// takes chunks t, t+T, ..., each wavefront butterflies its partials and the wavefront sums are
+// added in wavefront order.  Because fp32 addition is commutative, every lane ends with the same
+// bits, and the tree depends only on C and VEC (the input element size) -- not on the number of
+// rows, the row's position or alignment, or whether the row was read once (kept in registers) or
+// several times.
 #pragma once
 
 #include <type_traits>
@@ -29,21 +32,33 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// 16 bytes at any element boundary: rows of an odd length start anywhere.  The GPU takes 16-byte
+// global loads and stores at any alignment (one more 64-byte segment per wavefront access), so
+// misaligned rows need no element-wise path.
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));
+typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
+
+__device__ __forceinline__ u32x4_t load_16(const void* p) { return *reinterpret_cast<const u32x4_any_t*>(p); }
+
+template <typename T>
+__device__ __forceinline__ void unpack_chunk(const u32x4_t& raw, float (&v)[16 / sizeof(T)]) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(raw[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = Num<T>::from_bits((raw[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+  }
+}
+
 // Chunk of VEC consecutive elements starting at column c0 of a contiguous row of `cols`
 // elements, as fp32; elements past the row end read as `fill`.
 template <typename T>
-__device__ __forceinline__ void load_row_chunk(const T* row, int64_t cols, int64_t c0, bool vec_ok,
-                                               float fill, float (&v)[16 / sizeof(T)]) {
+__device__ __forceinline__ void load_row_chunk(const T* row, int64_t cols, int64_t c0, float fill,
+                                               float (&v)[16 / sizeof(T)]) {
   constexpr int VEC = 16 / sizeof(T);
-  if (vec_ok && c0 + VEC <= cols) {
-    const u32x4_t raw = *reinterpret_cast<const u32x4_t*>(row + c0);
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(raw[e]);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = Num<T>::from_bits((raw[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-    }
+  if (c0 + VEC <= cols) {
+    unpack_chunk<T>(load_16(row + c0), v);
   } else {
 #pragma unroll
     for (int e = 0; e < VEC; ++e) v[e] = (c0 + e < cols) ? Num<T>::load(row + c0 + e) : fill;
@@ -51,22 +66,26 @@ __device__ __forceinline__ void load_row_chunk(const T* row, int64_t cols, int64
 }
 
 // Store N fp32 values at columns c0 .. c0+N-1 of a contiguous row (columns >= cols skipped).
-// vec_ok promises the row start is 16-byte aligned.  NT marks the vector stores non-temporal
-// (streaming outputs nobody reads back soon: measured 6-10 % faster for the softmax rows).
-template <typename V>
-__device__ __forceinline__ void vstore(V* p, const V& v, bool nt) {
-  if (nt) __builtin_nontemporal_store(v, p);
-  else *p = v;
+// NT marks the vector stores non-temporal (streaming outputs nobody reads back soon: measured
+// 6-10 % faster for the softmax rows).
+template <bool NT>
+__device__ __forceinline__ void store_16(void* p, const u32x4_t& v) {
+  if (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any_t*>(p));
+  else *reinterpret_cast<u32x4_any_t*>(p) = v;
+}
+template <bool NT>
+__device__ __forceinline__ void store_8(void* p, const u32x2_t& v) {
+  if (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x2_any_t*>(p));
+  else *reinterpret_cast<u32x2_any_t*>(p) = v;
 }
 template <typename T, int N, bool NT = false>
-__device__ __forceinline__ void store_row_chunk(T* row, int64_t cols, int64_t c0, bool vec_ok,
-                                                const float (&v)[N]) {
-  if (vec_ok && c0 + N <= cols) {
+__device__ __forceinline__ void store_row_chunk(T* row, int64_t cols, int64_t c0, const float (&v)[N]) {
+  if (c0 + N <= cols) {
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
       for (int h = 0; h < N / 4; ++h) {
-        f32x4_t o = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
-        vstore(reinterpret_cast<f32x4_t*>(row + c0 + 4 * h), o, NT);
+        const f32x4_t o = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+        store_16<NT>(row + c0 + 4 * h, __builtin_bit_cast(u32x4_t, o));
       }
       return;
     } else {
@@ -79,11 +98,9 @@ __device__ __forceinline__ void store_row_chunk(T* row, int64_t cols, int64_t c0
           w[d] = (uint32_t)Num<T>::to_bits(v[2 * d]) | ((uint32_t)Num<T>::to_bits(v[2 * d + 1]) << 16);
       }
       if constexpr (N == 8) {
-        u32x4_t o = {w[0], w[1], w[2], w[3]};
-        vstore(reinterpret_cast<u32x4_t*>(row + c0), o, NT);
+        store_16<NT>(row + c0, u32x4_t{w[0], w[1], w[2], w[3]});
       } else {
-        u32x2_t o = {w[0], w[1]};
-        vstore(reinterpret_cast<u32x2_t*>(row + c0), o, NT);
+        store_8<NT>(row + c0, u32x2_t{w[0], w[1]});
       }
       return;
     }
@@ -104,8 +121,8 @@ __device__ __forceinline__ float soft_exp(float x, float shift, float shl2e) {
 }
 
 // ------------------------------------------------------------------ softmax rows ----
-// Row transform applied while loading scores (attention only): scale with the rounding of the
-// score dtype, then causal / boolean masking to -inf or an additive mask with rounding.
+// Row transform applied while loading attention scores: scale with the rounding of the score
+// dtype, then causal / boolean masking to -inf or an additive mask with rounding.
 struct AttnRow {
   float scale;
   int64_t col_limit;   // columns >= col_limit are causally masked (cols when not causal)
@@ -114,37 +131,34 @@ struct AttnRow {
   int mask_kind;       // 0 none, 1 bool, 2 additive (same dtype as the scores)
 };
 
-enum { kSoftmax = 0, kLogSoftmax = 1, kAttn = 2 };
+enum { kSoftmax = 0, kLogSoftmax = 1 };
 
-template <typename Tin, int MODE>
+template <typename T>
 __device__ __forceinline__ void transform_chunk(const AttnRow& ar, int64_t c0, int64_t cols,
-                                                float (&v)[16 / sizeof(Tin)]) {
-  if constexpr (MODE == kAttn) {
-    constexpr int VEC = 16 / sizeof(Tin);
+                                                float (&v)[16 / sizeof(T)]) {
+  constexpr int VEC = 16 / sizeof(T);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const int64_t c = c0 + e;
-      if (c >= cols) { v[e] = -INFINITY; continue; }
-      float s = Num<Tin>::round(v[e] * ar.scale);
-      if (c >= ar.col_limit) {
-        s = -INFINITY;
-      } else if (ar.mask_kind == 1) {
-        if (!reinterpret_cast<const uint8_t*>(ar.mask)[c * ar.mask_stride]) s = -INFINITY;
-      } else if (ar.mask_kind == 2) {
-        s = Num<Tin>::round(s + Num<Tin>::load(reinterpret_cast<const Tin*>(ar.mask) + c * ar.mask_stride));
-      }
-      v[e] = s;
+  for (int e = 0; e < VEC; ++e) {
+    const int64_t c = c0 + e;
+    if (c >= cols) { v[e] = -INFINITY; continue; }
+    float s = Num<T>::round(v[e] * ar.scale);
+    if (c >= ar.col_limit) {
+      s = -INFINITY;
+    } else if (ar.mask_kind == 1) {
+      if (!reinterpret_cast<const uint8_t*>(ar.mask)[c * ar.mask_stride]) s = -INFINITY;
+    } else if (ar.mask_kind == 2) {
+      s = Num<T>::round(s + Num<T>::load(reinterpret_cast<const T*>(ar.mask) + c * ar.mask_stride));
     }
+    v[e] = s;
   }
 }
 
-// Softmax / log-softmax of one row by one wavefront.  Reference semantics
-// (batch_invariant_ops.py:1074-1114, 974-1034): m = max; softmax = exp(x-m)/sum exp(x-m), with
-// an all -inf row giving 0; log_softmax = x - m - log(sum exp(x-m)).
-template <typename Tin, typename Tout, int MODE>
-__device__ __forceinline__ void softmax_row(const Tin* in, Tout* out, int64_t cols, bool vin,
-                                            bool vout, const AttnRow& ar) {
-  constexpr int VEC = 16 / sizeof(Tin);
+// In-place softmax of one row of attention scores by one wavefront.  Reference semantics
+// (batch_invariant_ops.py:1074-1114): m = max; softmax = exp(x-m)/sum exp(x-m), with an all -inf
+// row giving 0.
+template <typename T>
+__device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const AttnRow& ar) {
+  constexpr int VEC = 16 / sizeof(T);
   const int lane = threadIdx.x & 63;
   const int64_t nchunks = cdiv(cols, VEC);
   const bool fits = nchunks <= 64 * kRowRegChunks;
@@ -156,8 +170,8 @@ __device__ __forceinline__ void softmax_row(const Tin* in, Tout* out, int64_t co
     for (int j = 0; j < kRowRegChunks; ++j) {
       const int64_t ci = lane + 64 * j;
       if (ci < nchunks) {
-        load_row_chunk<Tin>(in, cols, ci * VEC, vin, -INFINITY, cache[j]);
-        transform_chunk<Tin, MODE>(ar, ci * VEC, cols, cache[j]);
+        load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, cache[j]);
+        transform_chunk<T>(ar, ci * VEC, cols, cache[j]);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) mx = fmaxf(mx, cache[j][e]);
       }
@@ -165,15 +179,15 @@ __device__ __forceinline__ void softmax_row(const Tin* in, Tout* out, int64_t co
   } else {
     for (int64_t ci = lane; ci < nchunks; ci += 64) {
       float v[VEC];
-      load_row_chunk<Tin>(in, cols, ci * VEC, vin, -INFINITY, v);
-      transform_chunk<Tin, MODE>(ar, ci * VEC, cols, v);
+      load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
+      transform_chunk<T>(ar, ci * VEC, cols, v);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) mx = fmaxf(mx, v[e]);
     }
   }
   mx = wave_max(mx);
   const bool all_neg_inf = (mx == -INFINITY);
-  const float shift = (MODE == kLogSoftmax || !all_neg_inf) ? mx : 0.f;
+  const float shift = all_neg_inf ? 0.f : mx;
   const float shl2e = shift * kLog2e;
 
   float sum = 0.f;
@@ -184,72 +198,48 @@ __device__ __forceinline__ void softmax_row(const Tin* in, Tout* out, int64_t co
       if (ci < nchunks) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          const float ex = (MODE != kLogSoftmax && all_neg_inf) ? 0.f : soft_exp<Tout>(cache[j][e], shift, shl2e);
-          if (MODE != kLogSoftmax) cache[j][e] = ex;
-          if (ci * VEC + e < cols) sum += ex;
+          cache[j][e] = all_neg_inf ? 0.f : soft_exp<T>(cache[j][e], shift, shl2e);
+          if (ci * VEC + e < cols) sum += cache[j][e];
         }
       }
     }
   } else {
     for (int64_t ci = lane; ci < nchunks; ci += 64) {
       float v[VEC];
-      load_row_chunk<Tin>(in, cols, ci * VEC, vin, -INFINITY, v);
-      transform_chunk<Tin, MODE>(ar, ci * VEC, cols, v);
+      load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
+      transform_chunk<T>(ar, ci * VEC, cols, v);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        const float ex = (MODE != kLogSoftmax && all_neg_inf) ? 0.f : soft_exp<Tout>(v[e], shift, shl2e);
+        const float ex = all_neg_inf ? 0.f : soft_exp<T>(v[e], shift, shl2e);
         if (ci * VEC + e < cols) sum += ex;
       }
     }
   }
   sum = wave_sum(sum);
 
-  if (MODE == kLogSoftmax) {
-    const float lse = logf(sum);
-    auto emit = [&](int64_t ci, float (&v)[VEC]) {
-      float o[VEC];
+  const bool zero = (sum == 0.f);
+  const float inv = zero ? 0.f : 1.0f / sum;
+  if (fits) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) o[e] = v[e] - mx - lse;
-      store_row_chunk<Tout, VEC>(out, cols, ci * VEC, vout, o);
-    };
-    if (fits) {
+    for (int j = 0; j < kRowRegChunks; ++j) {
+      const int64_t ci = lane + 64 * j;
+      if (ci < nchunks) {
+        float o[VEC];
 #pragma unroll
-      for (int j = 0; j < kRowRegChunks; ++j) {
-        const int64_t ci = lane + 64 * j;
-        if (ci < nchunks) emit(ci, cache[j]);
-      }
-    } else {
-      for (int64_t ci = lane; ci < nchunks; ci += 64) {
-        float v[VEC];
-        load_row_chunk<Tin>(in, cols, ci * VEC, vin, -INFINITY, v);
-        emit(ci, v);
+        for (int e = 0; e < VEC; ++e) o[e] = zero ? 0.f : cache[j][e] * inv;
+        store_row_chunk<T, VEC>(row, cols, ci * VEC, o);
       }
     }
   } else {
-    const bool zero = (sum == 0.f);
-    const float inv = zero ? 0.f : 1.0f / sum;
-    if (fits) {
+    for (int64_t ci = lane; ci < nchunks; ci += 64) {
+      float v[VEC];
+      load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
+      transform_chunk<T>(ar, ci * VEC, cols, v);
+      float o[VEC];
 #pragma unroll
-      for (int j = 0; j < kRowRegChunks; ++j) {
-        const int64_t ci = lane + 64 * j;
-        if (ci < nchunks) {
-          float o[VEC];
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) o[e] = zero ? 0.f : cache[j][e] * inv;
-          store_row_chunk<Tout, VEC>(out, cols, ci * VEC, vout, o);
-        }
-      }
-    } else {
-      for (int64_t ci = lane; ci < nchunks; ci += 64) {
-        float v[VEC];
-        load_row_chunk<Tin>(in, cols, ci * VEC, vin, -INFINITY, v);
-        transform_chunk<Tin, MODE>(ar, ci * VEC, cols, v);
-        float o[VEC];
-#pragma unroll
-        for (int e = 0; e < VEC; ++e)
-          o[e] = zero ? 0.f : (all_neg_inf ? 0.f : soft_exp<Tout>(v[e], shift, shl2e)) * inv;
-        store_row_chunk<Tout, VEC>(out, cols, ci * VEC, vout, o);
-      }
+      for (int e = 0; e < VEC; ++e)
+        o[e] = zero ? 0.f : (all_neg_inf ? 0.f : soft_exp<T>(v[e], shift, shl2e)) * inv;
+      store_row_chunk<T, VEC>(row, cols, ci * VEC, o);
     }
   }
 }
@@ -260,8 +250,7 @@ __device__ __forceinline__ void softmax_row(const Tin* in, Tout* out, int64_t co
 // reduction order are those of softmax_row.  Rows r >= nrows are skipped.
 template <typename Tin, typename Tout, int MODE, int R, int NC>
 __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, Tout* out, int64_t ld_out,
-                                                 int nrows, int64_t cols, bool vin, bool vout) {
-  static_assert(MODE != kAttn, "plain rows only");
+                                                 int nrows, int64_t cols) {
   static_assert(NC <= kRowRegChunks, "register cache");
   constexpr int VEC = 16 / sizeof(Tin);
   const int lane = threadIdx.x & 63;
@@ -274,7 +263,7 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
     for (int j = 0; j < NC; ++j) {
       const int64_t ci = lane + 64 * j;
       if (r < nrows && ci < nchunks) {
-        load_row_chunk<Tin>(in + r * ld_in, cols, ci * VEC, vin, -INFINITY, cache[r][j]);
+        load_row_chunk<Tin>(in + r * ld_in, cols, ci * VEC, -INFINITY, cache[r][j]);
       } else {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) cache[r][j][e] = -INFINITY;
@@ -333,7 +322,7 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
           float o[VEC];
 #pragma unroll
           for (int e = 0; e < VEC; ++e) o[e] = cache[r][j][e] - mx[r] - lse;
-          store_row_chunk<Tout, VEC, true>(orow, cols, ci * VEC, vout, o);
+          store_row_chunk<Tout, VEC, true>(orow, cols, ci * VEC, o);
         }
       }
     } else {
@@ -346,7 +335,7 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
           float o[VEC];
 #pragma unroll
           for (int e = 0; e < VEC; ++e) o[e] = zero ? 0.f : cache[r][j][e] * inv;
-          store_row_chunk<Tout, VEC, true>(orow, cols, ci * VEC, vout, o);
+          store_row_chunk<Tout, VEC, true>(orow, cols, ci * VEC, o);
         }
       }
     }

@@ -10,22 +10,158 @@ struct SoftmaxArgs {
   const void* in;
   void* out;
   int64_t rows, cols, ld_in, ld_out;
-  int32_t vin, vout;
 };
 
-// One wavefront per row for long rows.  Rows of at most 64*NC chunks (NC = 1, 2, 4 per lane):
-// fit_rows<NC>() rows per wavefront, whose loads are all issued before the first reduction,
-// with non-temporal output stores.  Same arithmetic per row either way.
-template <typename Tin, typename Tout, int MODE>
-__global__ __launch_bounds__(256) void softmax_kernel(SoftmaxArgs a) {
-  const int64_t r = (int64_t)blockIdx.x * kRowWaves + (threadIdx.x >> 6);
-  if (r >= a.rows) return;
-  AttnRow ar{1.f, a.cols, nullptr, 0, 0};
-  softmax_row<Tin, Tout, MODE>(reinterpret_cast<const Tin*>(a.in) + r * a.ld_in,
-                               reinterpret_cast<Tout*>(a.out) + r * a.ld_out, a.cols, a.vin != 0,
-                               a.vout != 0, ar);
+// Sum and maximum over a workgroup of NW wavefronts (each wavefront's butterfly, then the
+// wavefront results in wavefront order); every thread returns the same bits.  `part` holds NW
+// floats and may be reused after the next barrier.
+template <int NW>
+__device__ __forceinline__ float block_sum(float v, float* part) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float s = part[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) s += part[i];
+  return s;
+}
+template <int NW>
+__device__ __forceinline__ float block_max(float v, float* part) {
+  v = wave_max(v);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float s = part[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) s = fmaxf(s, part[i]);
+  return s;
 }
 
+// Rows longer than a wavefront's registers (over 256 chunks): one workgroup of T threads per
+// row, thread t holding chunks t, t + T, ... (NC of them, all loads issued before the first
+// reduction), so the row is read from memory once.  LOOP: rows past the register file of 1024
+// threads, read three times in groups of NC chunks per thread.  Bound by the row's read and
+// write; one wavefront per row, as the shorter rows have, leaves most of the chip idle at the row
+// counts of a decoding batch.  The same rule for every row count: the tree may depend on the row
+// length only.  MI355X, one wavefront per row with element-wise loads of misaligned rows ->
+// this: log-softmax [32, 50257] fp32 217 -> 13.2 us, softmax [64, 32000] bf16 57 -> 8.5 us,
+// [4096, 8192] bf16 44.3 -> 22.8 us (5.9 TB/s of read + write), [1, 131072] fp32 376 -> 38 us.
+template <typename Tin, typename Tout, int MODE, int T, int NC, bool LOOP>
+__global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
+  constexpr int VEC = 16 / sizeof(Tin);
+  constexpr int NW = T / 64;
+  __shared__ float part[2][NW];
+  const int64_t r = blockIdx.x;
+  const int t = threadIdx.x;
+  const Tin* in = reinterpret_cast<const Tin*>(a.in) + r * a.ld_in;
+  Tout* out = reinterpret_cast<Tout*>(a.out) + r * a.ld_out;
+  const int64_t cols = a.cols, nchunks = cdiv(cols, VEC);
+  const int64_t groups = LOOP ? cdiv(nchunks, T * NC) : 1;
+
+  // Chunk of group g held in slot j, and its raw bits; columns past the row end read as -inf.
+  auto chunk = [&](int64_t g, int j) { return t + T * (g * NC + j); };
+  constexpr uint32_t kNegInf = sizeof(Tin) == 4 ? 0xff800000u : (std::is_same<Tin, bf16_t>::value ? 0xff80ff80u : 0xfc00fc00u);
+  u32x4_t raw[NC];
+  auto load = [&](int64_t g) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int64_t c0 = chunk(g, j) * VEC;
+      raw[j] = u32x4_t{kNegInf, kNegInf, kNegInf, kNegInf};
+      if (c0 + VEC <= cols) {
+        raw[j] = load_16(in + c0);
+      } else if (c0 < cols) {
+#pragma unroll
+        for (int e = 0; e < VEC - 1; ++e) {
+          if (c0 + e < cols) {
+            if constexpr (sizeof(Tin) == 4) {
+              raw[j][e] = __float_as_uint(in[c0 + e]);
+            } else {
+              const uint32_t x = reinterpret_cast<const uint16_t*>(in)[c0 + e];
+              raw[j][e >> 1] = (e & 1) ? (raw[j][e >> 1] & 0xffffu) | (x << 16) : (raw[j][e >> 1] & 0xffff0000u) | x;
+            }
+          }
+        }
+      }
+    }
+  };
+  // Redefines the 16-bit rows' registers, so that the compiler unpacks them again instead of
+  // keeping the fp32 values of a whole row across a reduction (it spilled at NC = 16).
+  auto keep_raw = [&]() {
+    if constexpr (!LOOP && sizeof(Tin) == 2) {
+#pragma unroll
+      for (int j = 0; j < NC; ++j) asm volatile("" : "+v"(raw[j]));
+    }
+  };
+  // exp of a column past the row end is 0 (NaN only where the whole row gives NaN)
+  auto exps = [&](float (&v)[VEC], bool neg_inf, float shift, float shl2e) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+      v[e] = (MODE != kLogSoftmax && neg_inf) ? 0.f : soft_exp<Tout>(v[e], shift, shl2e);
+  };
+
+  float mx = -INFINITY;
+  for (int64_t g = 0; g < groups; ++g) {
+    load(g);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      float v[VEC];
+      unpack_chunk<Tin>(raw[j], v);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) mx = fmaxf(mx, v[e]);
+    }
+  }
+  mx = block_max<NW>(mx, part[0]);
+  keep_raw();
+  const bool neg_inf = (mx == -INFINITY);
+  const float shift = (MODE == kLogSoftmax || !neg_inf) ? mx : 0.f;
+  const float shl2e = shift * kLog2e;
+
+  // fp32 softmax of a resident row keeps the exponentials in the row's registers
+  constexpr bool kKeepExp = !LOOP && sizeof(Tin) == 4 && MODE == kSoftmax;
+  float sum = 0.f;
+  for (int64_t g = 0; g < groups; ++g) {
+    if constexpr (LOOP) load(g);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      float v[VEC];
+      unpack_chunk<Tin>(raw[j], v);
+      exps(v, neg_inf, shift, shl2e);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) sum += v[e];
+      if constexpr (kKeepExp) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) raw[j][e] = __float_as_uint(v[e]);
+      }
+    }
+  }
+  sum = block_sum<NW>(sum, part[1]);
+  keep_raw();
+
+  const bool zero = (sum == 0.f);
+  const float inv = zero ? 0.f : 1.0f / sum;
+  const float lse = MODE == kLogSoftmax ? logf(sum) : 0.f;
+  for (int64_t g = 0; g < groups; ++g) {
+    if constexpr (LOOP) load(g);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int64_t ci = chunk(g, j);
+      if (ci >= nchunks) continue;
+      float v[VEC];
+      unpack_chunk<Tin>(raw[j], v);
+      if constexpr (MODE == kLogSoftmax) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[e] = v[e] - mx - lse;
+      } else {
+        if constexpr (!kKeepExp) exps(v, neg_inf, shift, shl2e);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[e] = zero ? 0.f : v[e] * inv;
+      }
+      store_row_chunk<Tout, VEC, true>(out, cols, ci * VEC, v);
+    }
+  }
+}
+
+// Rows of at most 64*NC chunks (NC = 1, 2, 4 per lane): fit_rows<NC>() rows per wavefront, whose
+// loads are all issued before the first reduction, with non-temporal output stores.
 // Rows per wavefront R for rows of NC chunks per lane: two rows of one chunk, else one row
 // (measured on 512 MiB of bf16 rows: more rows per wavefront left fewer wavefronts in flight).
 template <int NC>
@@ -39,7 +175,7 @@ __global__ __launch_bounds__(256) void softmax_fit_kernel(SoftmaxArgs a) {
   const int n = a.rows - r < R ? (int)(a.rows - r) : R;
   softmax_rows_fit<Tin, Tout, MODE, R, NC>(reinterpret_cast<const Tin*>(a.in) + r * a.ld_in, a.ld_in,
                                            reinterpret_cast<Tout*>(a.out) + r * a.ld_out, a.ld_out, n,
-                                           a.cols, a.vin != 0, a.vout != 0);
+                                           a.cols);
 }
 
 template <typename Tin, typename Tout, int NC>
@@ -53,6 +189,16 @@ static int launch_softmax_fit(const SoftmaxArgs& a, int is_log, hipStream_t s) {
   return check_launch("softmax_fit_kernel");
 }
 
+template <typename Tin, typename Tout, int T, int NC, bool LOOP = false>
+static int launch_softmax_block(const SoftmaxArgs& a, int is_log, hipStream_t s) {
+  if (a.rows > 0x7fffffffLL) return fail(BIOPS_ERR_ARG, "too many rows");
+  if (is_log)
+    hipLaunchKernelGGL((softmax_block_kernel<Tin, Tout, kLogSoftmax, T, NC, LOOP>), dim3((unsigned)a.rows), dim3(T), 0, s, a);
+  else
+    hipLaunchKernelGGL((softmax_block_kernel<Tin, Tout, kSoftmax, T, NC, LOOP>), dim3((unsigned)a.rows), dim3(T), 0, s, a);
+  return check_launch("softmax_block_kernel");
+}
+
 template <typename Tin, typename Tout>
 static int launch_softmax(const SoftmaxArgs& a, int is_log, hipStream_t s) {
   constexpr int VEC = 16 / (int)sizeof(Tin);
@@ -60,28 +206,25 @@ static int launch_softmax(const SoftmaxArgs& a, int is_log, hipStream_t s) {
   if (nchunks <= 64) return launch_softmax_fit<Tin, Tout, 1>(a, is_log, s);
   if (nchunks <= 128) return launch_softmax_fit<Tin, Tout, 2>(a, is_log, s);
   if (nchunks <= 256) return launch_softmax_fit<Tin, Tout, 4>(a, is_log, s);
-  const int64_t blocks = cdiv(a.rows, kRowWaves);
-  if (blocks > 0x7fffffffLL) return fail(BIOPS_ERR_ARG, "too many rows");
-  if (is_log)
-    hipLaunchKernelGGL((softmax_kernel<Tin, Tout, kLogSoftmax>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((softmax_kernel<Tin, Tout, kSoftmax>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  return check_launch("softmax_kernel");
+  if (nchunks <= 1024) return launch_softmax_block<Tin, Tout, 256, 4>(a, is_log, s);
+  if (nchunks <= 4096) return launch_softmax_block<Tin, Tout, 1024, 4>(a, is_log, s);
+  if (nchunks <= 8192) return launch_softmax_block<Tin, Tout, 1024, 8>(a, is_log, s);
+  if (nchunks <= 16384) return launch_softmax_block<Tin, Tout, 1024, 16>(a, is_log, s);
+  return launch_softmax_block<Tin, Tout, 1024, 8, true>(a, is_log, s);
 }
 
 // ------------------------------------------------------------------ reductions ----
-// Contiguous rows (K == 1).  Rows of up to kWaveRowMax elements: one wavefront per row with the
-// tree described in rowops.h.  Longer rows: one 256-thread workgroup per row -- lane L of 256
-// takes chunks L, L+256, ...; each wavefront butterflies its 64 partials and the four wavefront
-// sums are added as (w0 + w1) + (w2 + w3).  The choice depends on N only; rows of up to 512
-// aligned 16-byte chunks go to reduce_rows_fit, which gives reduce_rows_wave's bits.
-constexpr int64_t kWaveRowMax = 65536;
+// Contiguous rows (K == 1).  Rows of up to kWaveRowChunks 16-byte chunks: one wavefront per row
+// with the tree described in rowops.h (reduce_rows_fit when the row is whole chunks, else
+// reduce_rows_wave; same bits).  Longer rows: one workgroup per row, of 256 threads up to
+// kBlock256Chunks chunks and of 1024 beyond.  The choice depends on N only.
+constexpr int64_t kWaveRowChunks = 512;
+constexpr int64_t kBlock256Chunks = 2048;
 
 struct ReduceArgs {
   const void* in;
   void* out;
   int64_t M, N, K, sM, sN, sK;
-  int32_t vin;   // contiguous rows are 16-byte aligned
   int32_t kvec;  // K > 1: k contiguous and every (m, n) row start 16-byte aligned
 };
 
@@ -108,7 +251,7 @@ __global__ __launch_bounds__(256) void reduce_rows_wave(ReduceArgs a) {
   float acc = 0.f;
   for (int64_t ci = lane; ci < nchunks; ci += 64) {
     float v[VEC];
-    load_row_chunk<Tin>(row, a.N, ci * VEC, a.vin != 0, 0.f, v);
+    load_row_chunk<Tin>(row, a.N, ci * VEC, 0.f, v);
 #pragma unroll
     for (int e = 0; e < VEC; ++e)
       if (ci * VEC + e < a.N) acc = reduce_add<OP>(acc, v[e]);
@@ -134,7 +277,7 @@ __global__ __launch_bounds__(256) void reduce_rows_fit(ReduceArgs a) {
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
     const int ci = lane + 64 * j;
-    raw[j] = ci < nchunks ? *reinterpret_cast<const u32x4_t*>(row + (int64_t)ci * VEC) : u32x4_t{0u, 0u, 0u, 0u};
+    raw[j] = ci < nchunks ? load_16(row + (int64_t)ci * VEC) : u32x4_t{0u, 0u, 0u, 0u};
   }
   float acc = 0.f;
 #pragma unroll
@@ -153,29 +296,42 @@ __global__ __launch_bounds__(256) void reduce_rows_fit(ReduceArgs a) {
   if (lane == 0) Num<Tout>::store(reinterpret_cast<Tout*>(a.out) + r, reduce_final<OP>(acc, a.N));
 }
 
-template <typename Tin, typename Tout, int OP>
-__global__ __launch_bounds__(256) void reduce_rows_block(ReduceArgs a) {
+// One workgroup of T threads per row: thread t adds chunks t, t + T, ... in order, kBlockUnroll
+// loads in flight, then the wavefronts' butterflies in wavefront order.  A row is one compute
+// unit's stream, so what bounds a few long rows is the loads that unit keeps in flight (one
+// wavefront per row takes 34.4 us for [2, 50000] fp32, a workgroup 7.7; [512, 65536] bf16 53.5 and
+// 11.8 us).
+constexpr int kBlockUnroll = 4;
+
+template <typename Tin, typename Tout, int OP, int T>
+__global__ __launch_bounds__(T) void reduce_rows_block(ReduceArgs a) {
   constexpr int VEC = 16 / sizeof(Tin);
-  __shared__ float part[4];
+  constexpr int NW = T / 64;
+  __shared__ float part[NW];
   const int64_t r = blockIdx.x;
   const int t = threadIdx.x;
   const Tin* row = reinterpret_cast<const Tin*>(a.in) + r * a.sM;
-  const int64_t nchunks = cdiv(a.N, VEC);
+  const int64_t whole = a.N / VEC;  // chunks inside the row
   float acc = 0.f;
-  for (int64_t ci = t; ci < nchunks; ci += 256) {
+  auto add = [&](const u32x4_t& raw) {
     float v[VEC];
-    load_row_chunk<Tin>(row, a.N, ci * VEC, a.vin != 0, 0.f, v);
+    unpack_chunk<Tin>(raw, v);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e)
-      if (ci * VEC + e < a.N) acc = reduce_add<OP>(acc, v[e]);
+    for (int e = 0; e < VEC; ++e) acc = reduce_add<OP>(acc, v[e]);
+  };
+  int64_t ci = t;
+  for (; ci + (kBlockUnroll - 1) * T < whole; ci += kBlockUnroll * T) {
+    u32x4_t raw[kBlockUnroll];
+#pragma unroll
+    for (int u = 0; u < kBlockUnroll; ++u) raw[u] = load_16(row + (ci + u * T) * VEC);
+#pragma unroll
+    for (int u = 0; u < kBlockUnroll; ++u) add(raw[u]);
   }
-  acc = wave_sum(acc);
-  if ((t & 63) == 0) part[t >> 6] = acc;
-  __syncthreads();
-  if (t == 0) {
-    const float s = (part[0] + part[1]) + (part[2] + part[3]);
-    Num<Tout>::store(reinterpret_cast<Tout*>(a.out) + r, reduce_final<OP>(s, a.N));
-  }
+  for (; ci < whole; ci += T) add(load_16(row + ci * VEC));
+  if (ci == whole)  // the thread whose turn the partial chunk is
+    for (int64_t n = whole * VEC; n < a.N; ++n) acc = reduce_add<OP>(acc, Num<Tin>::load(row + n));
+  const float s = block_sum<NW>(acc, part);
+  if (t == 0) Num<Tout>::store(reinterpret_cast<Tout*>(a.out) + r, reduce_final<OP>(s, a.N));
 }
 
 // Strided reduction (K > 1): a workgroup owns 64*VK consecutive k of one m (VK consecutive k
@@ -263,15 +419,17 @@ static int launch_reduce(const ReduceArgs& a, hipStream_t s) {
     constexpr int VEC = 16 / (int)sizeof(Tin);
     const int64_t blocks = cdiv(a.M, kRowWaves);
     const int64_t nc = cdiv(cdiv(a.N, VEC), 64);  // chunks per lane
-    if (a.vin && a.N % VEC == 0 && nc <= 8) {
+    if (a.N % VEC == 0 && nc <= kWaveRowChunks / 64) {
       if (nc <= 1) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 1>), dim3((unsigned)blocks), dim3(256), 0, s, a);
       else if (nc <= 2) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 2>), dim3((unsigned)blocks), dim3(256), 0, s, a);
       else if (nc <= 4) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 4>), dim3((unsigned)blocks), dim3(256), 0, s, a);
       else hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 8>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-    } else if (a.N <= kWaveRowMax) {
+    } else if (nc <= kWaveRowChunks / 64) {
       hipLaunchKernelGGL((reduce_rows_wave<Tin, Tout, OP>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+    } else if (nc <= kBlock256Chunks / 64) {
+      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP, 256>), dim3((unsigned)a.M), dim3(256), 0, s, a);
     } else {
-      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP>), dim3((unsigned)a.M), dim3(256), 0, s, a);
+      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP, 1024>), dim3((unsigned)a.M), dim3(1024), 0, s, a);
     }
   } else if (a.kvec) {
     constexpr int VK = 16 / (int)sizeof(Tin);
@@ -319,9 +477,7 @@ extern "C" int biops_softmax(int dtype_in, int dtype_out, int64_t rows, int64_t 
   if (rows < 0 || cols < 0) return fail(BIOPS_ERR_ARG, "negative size");
   if (rows == 0 || cols == 0) return BIOPS_OK;
   if (!in || !out) return fail(BIOPS_ERR_ARG, "null pointer");
-  SoftmaxArgs a{in, out, rows, cols, ld_in, ld_out, 0, 0};
-  a.vin = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && ((ld_in * dtype_bytes(dtype_in)) % 16 == 0);
-  a.vout = (reinterpret_cast<uintptr_t>(out) % 16 == 0) && ((ld_out * dtype_bytes(dtype_out)) % 16 == 0);
+  SoftmaxArgs a{in, out, rows, cols, ld_in, ld_out};
   BIOPS_DISPATCH_IN_OUT(dtype_in, dtype_out, launch_softmax, a, is_log, (hipStream_t)stream);
   return fail(BIOPS_ERR_DTYPE, "unsupported softmax dtype");
 }
@@ -336,10 +492,10 @@ extern "C" int biops_reduce(int op, int dtype_in, int dtype_out, int64_t M, int6
   if (M == 0 || K == 0) return BIOPS_OK;
   if (!in || !out) return fail(BIOPS_ERR_ARG, "null pointer");
   if (K == 1 && sN != 1 && N > 1) return fail(BIOPS_ERR_LAYOUT, "rows must be contiguous when K == 1");
-  ReduceArgs a{in, out, M, N, K, sM, sN, sK, 0, 0};
+  ReduceArgs a{in, out, M, N, K, sM, sN, sK, 0};
   const int elt = dtype_bytes(dtype_in);
-  a.vin = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && ((sM * elt) % 16 == 0);
-  a.kvec = K > 1 && sK == 1 && a.vin && ((sN * elt) % 16 == 0);
+  a.kvec = K > 1 && sK == 1 && (reinterpret_cast<uintptr_t>(in) % 16 == 0) && ((sM * elt) % 16 == 0) &&
+           ((sN * elt) % 16 == 0);
   if (M > 0x7fffffffLL) return fail(BIOPS_ERR_ARG, "too many rows");
   if (op == BIOPS_REDUCE_L2) {
     BIOPS_DISPATCH_IN_OUT(dtype_in, dtype_out, launch_reduce_op, BIOPS_REDUCE_L2, a, (hipStream_t)stream);

@@ -10,6 +10,7 @@ import torch.nn.functional as F
 import oracle
 from batch_invariant_ops import (
     linalg_vector_norm_batch_invariant,
+    log_softmax,
     mean_dim,
     set_batch_invariant_mode,
     softmax,
@@ -157,3 +158,51 @@ def test_mode_multi_dim_mean_matches_oracle():
         out_all = x.cuda().mean(dim=[])
     assert_close_scaled(out, oracle.mean_dims(x, (1, 3), keepdim=True), rel=1e-5, abs_scale=1e-7)
     assert_close_scaled(out_all, oracle.mean_dims(x, []), rel=1e-5, abs_scale=1e-7)
+
+
+# Row lengths in 16-byte chunks on both sides of every change of kernel (wavefront per row,
+# 256- / 1024-thread workgroups with 4, 8 and 16 chunks per thread, re-read rows).
+LONG_CHUNKS = (256, 257, 1024, 1025, 4096, 4097, 8192, 8193, 16384, 16385)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("chunks", LONG_CHUNKS)
+@pytest.mark.parametrize("extra", (0, 1))
+def test_long_rows_softmax_and_log_softmax(dtype, chunks, extra):
+    """Values against the oracle, a row alone, a misaligned copy of the rows (same bits), a row
+    of -inf and one with a single finite element.  ``rel``: one rounding of the output; the fp32
+    sums of both sides differ by far less (relative 2^-24 times the longest addition chain,
+    16 chunks x 8 elements + 10 levels, under 1e-5)."""
+    cols = chunks * (16 // torch.tensor([], dtype=dtype).element_size()) - extra * 3
+    x = randn(4, cols, seed=7300 + chunks, dtype=dtype, scale=3.0)
+    x[1] = -math.inf
+    x[2] = -math.inf
+    x[2, cols - 1] = 2.0
+    gx = x.cuda()
+    shifted = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")
+    shifted[1:] = gx.flatten()
+    for fn, ref, scale in ((softmax, oracle.softmax(x), 1e-7),
+                           (log_softmax, oracle.log_softmax(x), REL[dtype] * 8)):
+        out = fn(gx, -1)
+        assert_close_scaled(out, ref, rel=REL[dtype], abs_scale=scale, what=f"{fn.__name__} {cols}")
+        assert_bitwise(fn(gx[3:4], -1), out[3:4], "row 3 alone")
+        moved = fn(shifted[1:].view(4, cols), -1)
+        assert torch.equal(moved[::2], out[::2]) and torch.equal(moved[3], out[3])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("chunks", (512, 513, 2048, 2049, 20001))
+@pytest.mark.parametrize("extra", (0, 1))
+def test_long_rows_mean_and_norm(dtype, chunks, extra):
+    """Row lengths on both sides of every change of reduction kernel, as above."""
+    cols = chunks * (16 // torch.tensor([], dtype=dtype).element_size()) - extra
+    x = (randn(3, cols, seed=7400 + chunks, dtype=dtype) + 1.0).to(dtype)
+    gx = x.cuda()
+    shifted = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")
+    shifted[1:] = gx.flatten()
+    for fn, ref in ((mean_dim, oracle.mean_dim(x, -1)), (lambda t, d: linalg_vector_norm_batch_invariant(t, 2, d),
+                                                         x.double().square().sum(-1).sqrt())):
+        out = fn(gx, -1)
+        assert_close_scaled(out, ref, rel=REL[dtype], abs_scale=1e-7, what=f"{cols}")
+        assert_bitwise(fn(gx[1:2], -1), out[1:2], "row 1 alone")
+        assert_bitwise(fn(shifted[1:].view(3, cols), -1), out, "misaligned rows")
