@@ -235,6 +235,24 @@ int biops_sdpa_fused(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t 
                      const void* mask, int mask_dtype, int64_t mB, int64_t mH, int64_t mI, int64_t mJ,
                      int causal, float scale, void* out, void* stream);
 
+/* Same operator as biops_sdpa_fused without causal masking, for few query rows (lq <= 16) against
+ * more than 512 keys: the keys are split over workgroups, with 16-bit scores, row statistics and
+ * fp32 partial outputs in a workspace.  Same roundings; S is bitwise the materialised S, the row
+ * sum and the P V sum run in an order that depends on lk only.
+ * biops_sdpa_split_workspace_size: workspace bytes, or -1 when biops_sdpa_split does not take the
+ * call (dtype, head sizes, causal, query rows, key count).  The workspace is 256-byte aligned, out
+ * a contiguous [batch, hq, lq, dv]; layout conditions as biops_sdpa_fused.
+ * Replaces scaled_dot_product_attention_batch_invariant (batch_invariant_ops.py:1148-1213). */
+int64_t biops_sdpa_split_workspace_size(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t lq,
+                                        int64_t lk, int64_t d, int64_t dv, int causal);
+int biops_sdpa_split(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk,
+                     int64_t d, int64_t dv,
+                     const void* q, int64_t sqB, int64_t sqH, int64_t sqL,
+                     const void* k, int64_t skB, int64_t skH, int64_t skL,
+                     const void* v, int64_t svB, int64_t svH, int64_t svL,
+                     const void* mask, int mask_dtype, int64_t mB, int64_t mH, int64_t mI, int64_t mJ,
+                     float scale, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Tile order of biops_varlen_sdpa_fused: writes plan[5] entries (the plan's count of 128-row
  * query tiles) into the host array `order`, one per (sequence, query tile), as
  * (item << 32) | tile, sorted by the number of keys the tile sees under `causal`, most first

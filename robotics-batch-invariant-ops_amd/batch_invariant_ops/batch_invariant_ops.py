@@ -614,6 +614,10 @@ def _sdpa_glue(q4, k4, v4, group, mask4, scale, out_dtype):
     return bmm_persistent(probabilities.reshape(B * Hq, Lq, Lk), v4.reshape(B * Hq, Lk, v4.shape[-1]))
 
 
+# Query rows up to which biops_sdpa_split_workspace_size is asked (the library's own limit).
+_SPLIT_MAX_QUERY = 16
+
+
 def scaled_dot_product_attention_batch_invariant(
     query: torch.Tensor,
     key: torch.Tensor,
@@ -695,6 +699,22 @@ def scaled_dot_product_attention_batch_invariant(
     fused = _fused_attention_ok(query.dtype, D, Dv, q4, k4, v4)
     if fused and mask4 is not None:
         fused = bool(nat.load().biops_attention_fused_mask_ok(mask4.data_ptr(), mask_code, Lk, *mask4.stride()))
+    if fused and Lq <= _SPLIT_MAX_QUERY:
+        ws_bytes = _fast_fn("biops_sdpa_split_workspace_size")(
+            nat.dtype_code(query.dtype), B, Hq, Hkv, Lq, Lk, D, Dv, causal_code)
+        if ws_bytes >= 0:
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
+            rc = _fast_fn("biops_sdpa_split")(
+                nat.dtype_code(query.dtype), B, Hq, Hkv, Lq, Lk, D, Dv,
+                q4.data_ptr(), q4.stride(0), q4.stride(1), q4.stride(2),
+                k4.data_ptr(), k4.stride(0), k4.stride(1), k4.stride(2),
+                v4.data_ptr(), v4.stride(0), v4.stride(1), v4.stride(2),
+                mask4.data_ptr() if mask4 is not None else None, mask_code,
+                *(mask4.stride() if mask4 is not None else (0, 0, 0, 0)),
+                float(scale_value), out.data_ptr(), workspace.data_ptr(), ws_bytes, nat.stream_of(out),
+            )
+            nat.check(rc, "biops_sdpa_split")
+            return out.reshape(*leading, Lq, Dv)
     if fused:
         rc = _fast_fn("biops_sdpa_fused")(
             nat.dtype_code(query.dtype), B, Hq, Hkv, Lq, Lk, D, Dv,

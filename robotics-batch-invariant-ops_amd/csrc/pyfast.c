@@ -186,6 +186,31 @@ static PyObject* fast_sdpa_fused(PyObject* self, PyObject* const* args, Py_ssize
   return PyLong_FromLong(rc);
 }
 
+/* sdpa_split(dtype, batch, hq, hkv, lq, lk, d, dv, q, sqB, sqH, sqL, k, skB, skH, skL, v, svB,
+ *            svH, svL, mask, mask_dtype, mB, mH, mI, mJ, scale, out, workspace, bytes, stream) */
+static PyObject* fast_sdpa_split(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  int64_t iv[31];
+  void* pv[31];
+  float fv[31];
+  (void)self;
+  if (!parse(args, nargs, "llllllllplllplllplllplllllfpplp", iv, pv, fv)) return NULL;
+  int rc;
+  WITHOUT_GIL(rc, biops_sdpa_split((int)iv[0], iv[1], iv[2], iv[3], iv[4], iv[5], iv[6], iv[7], pv[8], iv[9],
+                                          iv[10], iv[11], pv[12], iv[13], iv[14], iv[15], pv[16], iv[17], iv[18],
+                                          iv[19], pv[20], (int)iv[21], iv[22], iv[23], iv[24], iv[25], fv[26],
+                                          pv[27], pv[28], iv[29], pv[30]));
+  return PyLong_FromLong(rc);
+}
+
+/* sdpa_split_workspace_size(dtype, batch, hq, hkv, lq, lk, d, dv, causal) -> bytes or -1 */
+static PyObject* fast_sdpa_split_workspace_size(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  int64_t iv[9];
+  (void)self;
+  if (!parse(args, nargs, "lllllllll", iv, NULL, NULL)) return NULL;
+  return PyLong_FromLongLong(biops_sdpa_split_workspace_size((int)iv[0], iv[1], iv[2], iv[3], iv[4], iv[5], iv[6],
+                                                             iv[7], (int)iv[8]));
+}
+
 /* copy_h2d(dst, src, bytes, stream) -> hipError_t: hipMemcpyAsync host -> device on `stream` */
 static PyObject* fast_copy_h2d(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   int64_t iv[4];
@@ -226,6 +251,9 @@ static PyMethodDef kMethods[] = {
     {"varlen_plan", (PyCFunction)(void (*)(void))fast_varlen_plan, METH_FASTCALL, "biops_varlen_plan"},
     {"varlen_fused_order", (PyCFunction)(void (*)(void))fast_varlen_fused_order, METH_FASTCALL,
      "biops_varlen_fused_order"},
+    {"sdpa_split", (PyCFunction)(void (*)(void))fast_sdpa_split, METH_FASTCALL, "biops_sdpa_split"},
+    {"sdpa_split_workspace_size", (PyCFunction)(void (*)(void))fast_sdpa_split_workspace_size, METH_FASTCALL,
+     "biops_sdpa_split_workspace_size"},
     {"varlen_sdpa_fused", (PyCFunction)(void (*)(void))fast_varlen_sdpa_fused, METH_FASTCALL,
      "biops_varlen_sdpa_fused"},
     {"varlen_sdpa_fused_planned", (PyCFunction)(void (*)(void))fast_varlen_sdpa_fused_planned, METH_FASTCALL,

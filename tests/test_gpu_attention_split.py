@@ -1,0 +1,149 @@
+"""Attention of few query rows against many keys (keys split over workgroups): parity with the CPU
+oracle and with the materialised path, bitwise batch invariance, and the rule that picks it.
+
+Parity as for the fused kernel (tests/_parity.py): the roundings are the same, only the fp32
+orders of the row sum and of the P V sum differ.
+"""
+
+import math
+
+import pytest
+import torch
+
+from batch_invariant_ops import scaled_dot_product_attention_batch_invariant as sdpa
+from batch_invariant_ops import _native as nat
+
+from _parity import check_sdpa, check_sdpa_against
+from _tol import assert_bitwise
+
+DTYPES16 = (torch.bfloat16, torch.float16)
+
+
+def randn(*shape, seed, dtype=torch.float32):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def size(B, Hq, Hkv, Lq, Lk, D=128, Dv=128, dtype=nat.BF16, causal=0):
+    return nat.load(require_gpu=False).biops_sdpa_split_workspace_size(dtype, B, Hq, Hkv, Lq, Lk, D, Dv, causal)
+
+
+def test_which_calls_are_split():
+    """By the sizes of one sample only: the batch size never changes the answer."""
+    for batch in (1, 3, 64):
+        assert size(batch, 16, 4, 1, 513) > 0 and size(batch, 16, 4, 16, 4096) > 0
+        assert size(batch, 16, 4, 1, 512) < 0 and size(batch, 16, 4, 17, 4096) < 0
+        assert size(batch, 16, 4, 1, 4096, causal=nat.CAUSAL_TOP_LEFT) < 0
+        assert size(batch, 16, 4, 1, 4096, dtype=nat.F32) < 0
+        assert size(batch, 16, 4, 1, 4096, D=264) < 0 and size(batch, 16, 4, 1, 4096, Dv=12) < 0
+    assert size(1, 16, 3, 1, 4096) < 0 and size(0, 16, 4, 1, 4096) < 0
+
+
+def test_argument_errors_come_before_any_launch():
+    lib = nat.load(require_gpu=False)
+    p = 256
+    need = size(1, 4, 4, 1, 600)
+
+    def call(dtype=nat.BF16, lk=600, q=p, sk=128, mask=None, mcode=0, ld=600, ws=p, nbytes=need):
+        return lib.biops_sdpa_split(dtype, 1, 4, 4, 1, lk, 128, 128, q, 0, 0, 128, p, 0, 0, sk, p, 0, 0, 128,
+                                    mask, mcode, 0, 0, ld, 1, 1.0, p, ws, nbytes, None)
+
+    assert call(dtype=nat.F32) == 1 and call(lk=100) == 1 and call(q=None) == 1
+    assert call(q=p + 2) == 2 and call(sk=130) == 2 and call(ws=p + 16) == 2
+    assert call(nbytes=need - 1) == 5
+    assert call(mask=p, mcode=nat.F32) == 3 and call(mask=p + 1, mcode=nat.BOOL) == 2
+
+
+SHAPES = (
+    # B, Hq, Hkv, Lq, Lk, D, Dv: packed rows 1, 4, 31, 32, 33, 64, 66 and 128; key counts around the 64-key
+    # wavefront, the 256-key workgroup and the value split (256 keys up to 2048, then 512)
+    (2, 1, 1, 1, 513, 128, 128),
+    (2, 16, 4, 1, 576, 128, 128),
+    (1, 1, 1, 16, 767, 64, 64),
+    (1, 31, 1, 1, 768, 64, 40),
+    (1, 4, 1, 8, 769, 72, 128),
+    (2, 6, 2, 11, 1000, 256, 256),
+    (1, 8, 2, 16, 2048, 128, 64),
+    (1, 12, 2, 11, 2049, 8, 200),
+    (1, 8, 1, 16, 2561, 128, 128),
+)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES16)
+@pytest.mark.parametrize("mask_kind", ("none", "boolean", "additive"))
+@pytest.mark.parametrize("shape", SHAPES)
+def test_split_sdpa_matches_oracle_and_materialized(dtype, mask_kind, shape, monkeypatch):
+    B, Hq, Hkv, Lq, Lk, D, Dv = shape
+    if mask_kind != "none":
+        Lk = -(-Lk // 4) * 4  # masks of other key counts take the materialised path
+    seed = 9000 + 10 * SHAPES.index(shape)
+    q = randn(B, Hq, Lq, D, seed=seed, dtype=dtype)
+    k = randn(B, Hkv, Lk, D, seed=seed + 1, dtype=dtype)
+    v = randn(B, Hkv, Lk, Dv, seed=seed + 2, dtype=dtype)
+    mask = None
+    if mask_kind != "none":
+        keep = torch.rand(B, 1, Lq, Lk, generator=torch.Generator().manual_seed(seed + 3)) > 0.2
+        keep[:, :, Lq // 2] = False  # a fully masked row gives 0
+        keep[0, :, :, : Lk // 2] = False  # whole workgroups without a visible key
+        mask = keep
+        if mask_kind == "additive":
+            mask = (torch.rand(B, 1, Lq, Lk, generator=torch.Generator().manual_seed(seed + 4)) * -10).to(dtype)
+            mask[~keep] = -math.inf
+    assert size(B, Hq, Hkv, Lq, Lk, D, Dv) > 0
+    kw = dict(enable_gqa=Hq != Hkv)
+    dev = dict(kw, attn_mask=None if mask is None else mask.cuda())
+    out = sdpa(q.cuda(), k.cuda(), v.cuda(), **dev)
+    check_sdpa(out, q, k, v, attn_mask=mask, what=f"split vs oracle {shape}", **kw)
+    if mask is not None:
+        assert torch.count_nonzero(out[:, :, Lq // 2]) == 0
+    monkeypatch.setenv("BIOPS_ATTENTION_MATERIALIZE", "1")
+    mat = sdpa(q.cuda(), k.cuda(), v.cuda(), **dev)
+    check_sdpa_against(out, mat, q, k, v, attn_mask=mask, min_exact=0.9, what="split vs materialised", **kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES16)
+@pytest.mark.parametrize("heads", ((16, 4, 1), (64, 8, 16), (8, 8, 5)))
+def test_split_sdpa_is_batch_invariant(dtype, heads):
+    """Samples alone and in a batch large enough for several row tiles per workgroup; the batch is
+    a view of a longer cache (row and batch strides of their own)."""
+    Hq, Hkv, Lq = heads
+    B, Lk = 9, 1111
+    q = randn(B, Lq, Hq, 128, seed=9200, dtype=dtype).cuda().transpose(1, 2)
+    kc = randn(B, Lk + 50, Hkv, 128, seed=9201, dtype=dtype).cuda()
+    vc = randn(B, Lk + 50, Hkv, 128, seed=9202, dtype=dtype).cuda()
+    k, v = kc[:, 7:7 + Lk].transpose(1, 2), vc[:, 7:7 + Lk].transpose(1, 2)
+    full = sdpa(q, k, v, enable_gqa=Hq != Hkv)
+    for j in (0, 4, 8):
+        one = slice(j, j + 1)
+        assert_bitwise(sdpa(q[one], k[one], v[one], enable_gqa=Hq != Hkv), full[one], f"sample {j} alone")
+        assert_bitwise(sdpa(q[one].contiguous(), k[one].contiguous(), v[one].contiguous(), enable_gqa=Hq != Hkv),
+                       full[one], f"sample {j} contiguous")
+
+
+@pytest.mark.gpu
+def test_split_sdpa_ignores_what_lies_past_the_keys():
+    """Key and value rows past the end (NaN here) reach no output."""
+    kc, vc = (torch.full((1, 2, 700, 64), math.nan, dtype=torch.bfloat16, device="cuda") for _ in "kv")
+    q = randn(1, 4, 2, 64, seed=9300, dtype=torch.bfloat16).cuda()
+    k, v = (randn(1, 2, 613, 64, seed=9301 + i, dtype=torch.bfloat16).cuda() for i in range(2))
+    kc[:, :, :613], vc[:, :, :613] = k, v
+    assert_bitwise(sdpa(q, kc[:, :, :613], vc[:, :, :613], enable_gqa=True), sdpa(q, k, v, enable_gqa=True), "")
+
+
+@pytest.mark.gpu
+def test_split_sdpa_in_a_graph():
+    q = randn(2, 8, 1, 128, seed=9400, dtype=torch.bfloat16).cuda()
+    k, v = (randn(2, 2, 2100, 128, seed=9401 + i, dtype=torch.bfloat16).cuda() for i in range(2))
+    sdpa(q, k, v, enable_gqa=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = sdpa(q, k, v, enable_gqa=True)
+    for seed in (9410, 9420, 9430):
+        q.copy_(randn(2, 8, 1, 128, seed=seed, dtype=torch.bfloat16))
+        k.copy_(randn(2, 2, 2100, 128, seed=seed + 1, dtype=torch.bfloat16))
+        eager = sdpa(q, k, v, enable_gqa=True)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_bitwise(out, eager, f"replay {seed}")
