@@ -28,6 +28,10 @@ struct BmmArgs {
   const void* B2;
   void* C;
   const void* bias;
+  // Plain epilogue, K-major B, no row groups: C row m of inner batch b2 becomes round(round(acc) + row_bias[b2*sR2 + m])
+  // (a convolution's channel bias, added after the GEMM's rounding); nullptr: none.
+  const void* row_bias;
+  int64_t sR2;
   int64_t M, N, K;
   int64_t lda, ldb, ldc;
   int64_t nb1, nb2, gB;

@@ -174,8 +174,11 @@ __device__ __forceinline__ void bmm_tile(const BmmArgs& args, uint32_t t, char* 
 
   T* Cp = reinterpret_cast<T*>(args.C) + b1 * args.sC1 + b2 * args.sC2 + m0 * args.ldc + n0;
   const T* bias = (EPI != kEpiSwiglu && args.bias) ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
-  Tile::template epilogue<EPI == kEpiSwiglu>(smem, acc, Cp, args.ldc, rows < BM ? (int)rows : BM,
-                                             cols < kCols ? (int)cols : kCols, bias, args.c_vec != 0);
+  constexpr bool kRowBias = EPI != kEpiSwiglu && BKM && !GRP;
+  const T* row_bias = (kRowBias && args.row_bias) ? reinterpret_cast<const T*>(args.row_bias) + b2 * args.sR2 + m0 : nullptr;
+  Tile::template epilogue<EPI == kEpiSwiglu, kRowBias>(smem, acc, Cp, args.ldc, rows < BM ? (int)rows : BM,
+                                                       cols < kCols ? (int)cols : kCols, bias, row_bias,
+                                                       args.c_vec != 0);
 }
 
 // Persistent entries walk tiles t = slot, slot + G, ... (slot = XCD-aware rank of the
@@ -231,7 +234,8 @@ __device__ __forceinline__ void skinny_store(const BmmArgs& args, const TileOrig
   T* Cp = reinterpret_cast<T*>(args.C) + o.b1 * args.sC1 + o.b2 * args.sC2 + (o.m0 + S::WR * wr) * args.ldc + n0;
   const T* bias = args.bias ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
   const int wrows = rows - S::WR * wr, wcols = cols - S::WC * wc;
-  S::Math::store(acc, Cp, args.ldc, wrows < S::WR ? wrows : S::WR, wcols < S::WC ? wcols : S::WC, bias);
+  const T* row_bias = args.row_bias ? reinterpret_cast<const T*>(args.row_bias) + o.b2 * args.sR2 + o.m0 + S::WR * wr : nullptr;
+  S::Math::store(acc, Cp, args.ldc, wrows < S::WR ? wrows : S::WR, wcols < S::WC ? wcols : S::WC, bias, row_bias);
 }
 
 // One 32 x BC (or 64 x BC) block per workgroup.
@@ -355,7 +359,8 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool skinny_ok, bool n
   if (forced == kSkinnyCfg && skinny_ok) return forced;
   // Four-wave entries: the skinny conditions (direct loads, K-major B, plain rows, no SwiGLU),
   // or the same with a 16-bit N-major B; 32-bit output offsets inside a 256-row tile.
-  const bool big_ok = (skinny_ok || (nmajor16 && !swiglu && !grouped)) && dtype != BIOPS_F32 &&
+  // Not built for a row bias.
+  const bool big_ok = a.row_bias == nullptr && (skinny_ok || (nmajor16 && !swiglu && !grouped)) && dtype != BIOPS_F32 &&
                       a.ldc < (int64_t(1) << 23);
   if (forced >= kBigCfg && forced < kBigEnd && big_ok) return forced;
   // The weight-streaming entries: grouped rows, 16-bit N-major B on the direct path.
@@ -851,7 +856,7 @@ __global__ __launch_bounds__(256) void grouped_kernel(GroupedArgs a) {
     Tile::mainloop(smem, acc, typename Tile::ARows{A, lda, rows}, avec, src, K);
     const bool cvec = al(C, 0) && (ldc * elt) % 16 == 0;
     Tile::template epilogue<false>(smem, acc, C, ldc, rows < BM ? (int)rows : BM,
-                                   cols < BN ? (int)cols : BN, nullptr, cvec);
+                                   cols < BN ? (int)cols : BN, nullptr, nullptr, cvec);
   }
 }
 

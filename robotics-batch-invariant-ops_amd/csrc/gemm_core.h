@@ -108,6 +108,21 @@ __device__ __forceinline__ float swiglu_value(float g_acc, float u_acc) {
   return Num<T>::round(g / (1.0f + expf(-g))) * u;
 }
 
+// round(x + b) of every element x of a 16-byte chunk.
+template <typename T>
+__device__ __forceinline__ u32x4_t add_round(u32x4_t v, float b) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    if constexpr (sizeof(T) == 4) {
+      v[d] = __float_as_uint(__uint_as_float(v[d]) + b);
+    } else {
+      const float lo = Num<T>::from_bits(v[d] & 0xffffu) + b, hi = Num<T>::from_bits(v[d] >> 16) + b;
+      v[d] = (uint32_t)Num<T>::to_bits(lo) | ((uint32_t)Num<T>::to_bits(hi) << 16);
+    }
+  }
+  return v;
+}
+
 // LDS tile layout: rows of 128 bytes (one K step), unpadded; 16-byte chunk c of row r lives in
 // slot c ^ ((r >> 1) & 7).  Sixteen consecutive rows reading the same chunk hit 16 distinct
 // (half-row, slot) bank groups, so the MFMA operand reads (ds_read_b128) are conflict-free.
@@ -639,12 +654,12 @@ struct GemmTile {
   // 16-byte stores.  SWIGLU: gate / up accumulators of one output sit in
   // blocks (i, j) / (i, j+1) of the same lane; the stored value is
   // round(round(silu(round(g))) * round(u)) and the tile is BN/2 wide.  Otherwise the value is
-  // round(acc + bias[col]) (bias may be null: no add).  Ends with a barrier, so the LDS ring
-  // is free for the next tile.
-  template <bool SWIGLU>
+  // round(acc + bias[col]) (bias may be null: no add), and with ROWB the written value is
+  // round(that + row_bias[row]) (row_bias may be null).  Ends with a barrier, so the LDS ring is free for the next tile.
+  template <bool SWIGLU, bool ROWB = false>
   __device__ static __forceinline__ void epilogue(char* smem, Acc (&acc)[FM][FN], T* C,
                                                   int64_t ldc, int rows, int cols, const T* bias,
-                                                  bool c_vec) {
+                                                  const T* row_bias, bool c_vec) {
     constexpr int OUTW = SWIGLU ? BN / 2 : BN;
     constexpr int PITCH = OUTW * (int)sizeof(T);
     constexpr int SWZ = OUTW / VEC >= 8 ? 7 : OUTW / VEC - 1;  // chunk swizzle stays inside the row
@@ -679,6 +694,19 @@ struct GemmTile {
       if (r >= rows || c0 >= cols) continue;
       const char* src = smem + r * PITCH + (((c0 / VEC) ^ (r & SWZ)) * 16);
       T* dst = C + (int64_t)r * ldc + c0;
+      if constexpr (ROWB) {
+        if (row_bias) {
+          const u32x4_t v = add_round<T>(*reinterpret_cast<const u32x4_t*>(src), Num<T>::load(row_bias + r));
+          if (c_vec && c0 + VEC <= cols) {
+            *reinterpret_cast<u32x4_t*>(dst) = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+              if (c0 + e < cols) dst[e] = reinterpret_cast<const T*>(&v)[e];
+          }
+          continue;
+        }
+      }
       if (c_vec && c0 + VEC <= cols) {
         *reinterpret_cast<u32x4_t*>(dst) = *reinterpret_cast<const u32x4_t*>(src);
       } else {

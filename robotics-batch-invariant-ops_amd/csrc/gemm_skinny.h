@@ -99,7 +99,8 @@ struct SkinnyMath<T, AR, BC, true> {
   }
   // round(acc (+ bias[n])) of this lane's outputs: row 16 i + 4 (l / 16) + r, column
   // 16 j + l % 16.
-  __device__ static __forceinline__ void store(const Acc& acc, T* C, int64_t ldc, int rows, int cols, const T* bias) {
+  __device__ static __forceinline__ void store(const Acc& acc, T* C, int64_t ldc, int rows, int cols, const T* bias,
+                                               const T* row_bias) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < CB; ++j) {
@@ -111,7 +112,11 @@ struct SkinnyMath<T, AR, BC, true> {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = 16 * i + 4 * (lane >> 4) + r;
-          if (row < rows) Num<T>::store(C + (int64_t)row * ldc + col, bias ? acc.c[i][j][r] + bv : acc.c[i][j][r]);
+          if (row < rows) {
+            float v = bias ? acc.c[i][j][r] + bv : acc.c[i][j][r];
+            if (row_bias) v = Num<T>::round(v) + Num<T>::load(row_bias + row);
+            Num<T>::store(C + (int64_t)row * ldc + col, v);
+          }
         }
     }
   }
@@ -144,7 +149,8 @@ struct SkinnyMath<T, AR, BC, false> {
   static constexpr int COUNT = 4;
   __device__ static __forceinline__ void one(Acc& acc, const Frags& f, int n) { Mfma<T>::step(acc.c, f.a[n], f.b[n]); }
   // Row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
-  __device__ static __forceinline__ void store(const Acc& acc, T* C, int64_t ldc, int rows, int cols, const T* bias) {
+  __device__ static __forceinline__ void store(const Acc& acc, T* C, int64_t ldc, int rows, int cols, const T* bias,
+                                               const T* row_bias) {
     const int lane = threadIdx.x & 63;
     const int col = lane & 31;
     if (col >= cols) return;
@@ -152,7 +158,11 @@ struct SkinnyMath<T, AR, BC, false> {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-      if (row < rows) Num<T>::store(C + (int64_t)row * ldc + col, bias ? acc.c[r] + bv : acc.c[r]);
+      if (row < rows) {
+        float v = bias ? acc.c[r] + bv : acc.c[r];
+        if (row_bias) v = Num<T>::round(v) + Num<T>::load(row_bias + row);
+        Num<T>::store(C + (int64_t)row * ldc + col, v);
+      }
     }
   }
 };

@@ -239,3 +239,37 @@ def test_conv_strided_input_and_edge_cases():
     tw = randn(6, 2, 3, 3, seed=7102, dtype=torch.bfloat16).cuda()
     with pytest.raises(AssertionError, match="non-overlapping"):
         conv_transpose2d_batch_invariant(x, tw, None, (2, 2), (0, 0), (1, 1), (0, 0), 1)
+
+
+# Patch rows around the 16-row steps of a unit, one and four steps per unit (the last shape), K in
+# whole GEMM steps (weights used in place) and not, groups, dilation, every tile path of the GEMM
+# (few rows: the skinny blocks; many: the table entries).
+PREP_SHAPES = (
+    # x, weight, stride, padding, dilation, groups
+    ((1, 3, 17, 17), (8, 3, 3, 3), 1, 0, 1, 1),
+    ((2, 64, 9, 15), (40, 64, 1, 1), 1, 0, 1, 1),
+    ((3, 8, 12, 11), (12, 4, 3, 2), 2, 1, 2, 2),
+    ((1, 64, 5, 13), (300, 64, 3, 3), 1, 1, 1, 1),
+    ((4, 16, 33, 31), (130, 16, 3, 3), 1, 2, 1, 1),
+    ((5, 48, 61, 67), (64, 48, 3, 3), 1, 1, 1, 1),
+)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("case", PREP_SHAPES)
+def test_conv2d_patches_and_channel_bias(dtype, case):
+    """Against the oracle; the bias is added to the rounded sum (bitwise: the call without bias plus
+    the bias); channels-last input gives the bits of the contiguous one."""
+    shape, wshape, stride, padding, dilation, groups = case
+    x = randn(*shape, seed=7300, dtype=dtype).cuda()
+    w = randn(*wshape, seed=7301, dtype=dtype, scale=0.2).cuda()
+    b = randn(wshape[0], seed=7302, dtype=dtype).cuda()
+
+    def conv(x, bias):
+        return conv2d_batch_invariant(x, w, bias, (stride,) * 2, (padding,) * 2, (dilation,) * 2, False, (0, 0), groups)
+
+    out = conv(x, b)
+    assert_conv_close(out, x, w, b, (stride,) * 2, (padding,) * 2, (dilation,) * 2, False, groups)
+    assert torch.equal(out, conv(x, None) + b.view(1, -1, 1, 1))
+    assert torch.equal(out, conv(x.to(memory_format=torch.channels_last), b))
+    assert torch.equal(out[:1], conv(x[:1], b))
