@@ -352,7 +352,35 @@ static bool cfg_ok(int dtype, int c, bool swiglu, bool grouped) {
   return !swiglu || c <= 2 || c == 7;
 }
 
-static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool skinny_ok, bool nmajor16) {
+// fp32 products on the direct path: microseconds of an entry as rounds x (K x per-K + fixed).  A
+// round is kF32Slots tiles per compute unit; an entry whose workgroups pair up on a unit (2 and
+// 4) is cheaper alone (kF32PerKAlone, up to one tile per unit).  fp32 tiles are bound by their MFMA
+// chains at every size (157 TF/s against 2.5 PF/s in 16 bits), so small tiles lose little and
+// save whole rounds, which the 16-bit rates below cannot express.  Per-K and fixed times fitted
+// on MI355X to 40 shapes (M 16-2048, K 64-4096, N 64-4096, batches to 128, both B layouts) with every
+// entry forced: the choice is within 1 % of the best entry on geometric average and within 12 %
+// everywhere; the 16-bit model was 7 % off (16 x 1024 x 576 x 576 152.9 -> 112 us, 1020 x 3936 x
+// 1044 162 -> 134, 408 x 768 x 4096 34.3 -> 31.1).
+static const int kF32Slots[kNumCfg] = {0, 1, 2, 1, 2, 2, 4, 0, 1, 0, 1, 1};
+static const double kF32PerK[kNumCfg] = {0, .115, .127, .033, .033, .0188, .0202, 0, .060, 0, .114, .1135};
+static const double kF32PerKAlone[kNumCfg] = {0, 0, .064, 0, .0183, 0, 0, 0, 0, 0, 0, 0};
+static const double kF32Fixed[kNumCfg] = {0, 5.2, 5.0, 3.2, 2.0, 2.2, 2.2, 0, 3.6, 0, 4.8, 4.8};
+static int pick_cfg_f32(const BmmArgs& a) {
+  const int cus = device_cus();
+  int best = 2;
+  double best_cost = 1e300;
+  for (int c = 0; c < kNumCfg; ++c) {
+    if (kF32Slots[c] == 0) continue;
+    const int64_t tiles = a.nb1 * a.nb2 * cdiv(a.M, kCfgBM[c]) * cdiv(a.N, kCfgBN[c]);
+    const bool alone = kF32PerKAlone[c] > 0 && tiles <= cus;
+    const double rounds = alone ? 1.0 : (double)cdiv(tiles, (int64_t)cus * kF32Slots[c]);
+    const double cost = rounds * ((double)a.K * (alone ? kF32PerKAlone[c] : kF32PerK[c]) + kF32Fixed[c]);
+    if (cost < best_cost) { best_cost = cost; best = c; }
+  }
+  return best;
+}
+
+static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skinny_ok, bool nmajor16) {
   const bool swiglu = epi == kEpiSwiglu;
   const bool grouped = a.grp != nullptr;
   const int forced = forced_cfg();
@@ -410,7 +438,10 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool skinny_ok, bool n
   // entries forced on one box: M = 512, N = 2048, K = 8192: 34.5 against 37.1 us for entry 6;
   // M = 256: 33.3 against 34.5; M = 128, N = 8192, K = 2048: 11.6 against 12.4; M = 64: 10.9
   // against 11.4).
-  if ((best == 4 || best == 6) && prefer32) best = (big_ok && !nmajor16) ? kBigCfg + 6 : 6;
+  // (fp32 on the direct path has its own model.)
+  const bool f32_direct = dtype == BIOPS_F32 && direct && !swiglu && !grouped;
+  if (f32_direct) best = pick_cfg_f32(a);
+  else if ((best == 4 || best == 6) && prefer32) best = (big_ok && !nmajor16) ? kBigCfg + 6 : 6;
   // The skinny entry: 32-column (or narrower) blocks in one round, or, with at least two row
   // blocks and K >= 1024, 64-column blocks in one round (MI355X, bf16, same-box A/B against the
   // automatic choice before them, same bits: 256 x 2048 x 8192 33.7 -> 26.8 us, 128 x 4096 x
@@ -420,8 +451,9 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool skinny_ok, bool n
   // of 32 or 64 columns in one round with 2 to 8 of them down M (512 x 2048 x 8192 38.4 ->
   // 33.0 us, 300 x 3000 x 2048 11.7 -> 10.3 us, 128 x 8192 x 2048 12.7 -> 12.2 us; 16 down M
   // lost: 1024 x 1024 x 4096 19.0 -> 19.8 us).
+  // fp32 takes it from K = 448 on (below that it was even with the table entries or lost: 58 x 96 x 472 7.7 against 6.4 us, 475 x 224 x 608 10.0 against 9.0).
   const int64_t row_blocks = batch * cdiv(a.M, 32), row_blocks64 = batch * cdiv(a.M, 64);
-  if (skinny_ok && (row_blocks * cdiv(a.N, 32) <= cus ||
+  if (skinny_ok && (dtype != BIOPS_F32 || a.K >= 448) && (row_blocks * cdiv(a.N, 32) <= cus ||
                     (row_blocks >= 2 && a.K >= 1024 && row_blocks * cdiv(a.N, 64) <= cus) ||
                     (dtype != BIOPS_F32 && row_blocks64 >= 2 && row_blocks64 <= 8 && a.K >= 1024 &&
                      row_blocks64 * cdiv(a.N, 64) <= cus)))
@@ -702,7 +734,7 @@ static int prepare_bmm(int dtype, BmmArgs& a, int epi, bool b_kmajor, bool& dire
   // Grouped rows run on the table entries only (the skinny and large-tile kernels take a fixed
   // tile count from the host); those two read K-major B only.
   const bool skinny_ok = direct && b_kmajor && epi != kEpiSwiglu && a.grp == nullptr;
-  return pick_cfg(dtype, a, epi, skinny_ok, direct && !b_kmajor && elt == 2);
+  return pick_cfg(dtype, a, epi, direct, skinny_ok, direct && !b_kmajor && elt == 2);
 }
 
 int grouped_tile_rows(int dtype, BmmArgs a, int epi, bool b_kmajor) {
