@@ -253,6 +253,23 @@ int biops_sdpa_split(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t 
                      const void* mask, int mask_dtype, int64_t mB, int64_t mH, int64_t mI, int64_t mJ,
                      float scale, void* out, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Same operator as biops_sdpa for float32 without a score matrix: one pass over the keys in blocks
+ * of 32, in order, probabilities and sums in float32, merged per 128 keys in order and divided by the
+ * row sum at the end.  biops_sdpa_f32_workspace_size: bytes that a launch with few query tiles needs
+ * to spread its keys over workgroups (0 otherwise, -1 for sizes it does not take; same bits either
+ * way), 256-byte aligned.  biops_sdpa_f32_supported: 1 when it takes the sizes (1 <= d, dv <= 128, multiples of 4).
+ * 16-byte aligned q / k / v / out, strides multiples of 4 elements, any mask strides, out a
+ * contiguous [batch, hq, lq, dv].
+ * Replaces scaled_dot_product_attention_batch_invariant (batch_invariant_ops.py:1148-1213). */
+int biops_sdpa_f32_supported(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t d, int64_t dv);
+int64_t biops_sdpa_f32_workspace_size(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t d, int64_t dv);
+int biops_sdpa_f32(int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk, int64_t d, int64_t dv,
+                   const void* q, int64_t sqB, int64_t sqH, int64_t sqL,
+                   const void* k, int64_t skB, int64_t skH, int64_t skL,
+                   const void* v, int64_t svB, int64_t svH, int64_t svL,
+                   const void* mask, int mask_dtype, int64_t mB, int64_t mH, int64_t mI, int64_t mJ,
+                   int causal, float scale, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Tile order of biops_varlen_sdpa_fused: writes plan[5] entries (the plan's count of 128-row
  * query tiles) into the host array `order`, one per (sequence, query tile), as
  * (item << 32) | tile, sorted by the number of keys the tile sees under `causal`, most first

@@ -393,8 +393,8 @@ extern "C" int biops_conv(int dtype, int nd, int transposed, int64_t batch, int6
     g.C = out; g.ldc = c.Lout; g.sC1 = c.Cout * c.Lout; g.sC2 = c.Og * c.Lout;
     g.M = c.Og; g.N = c.Lout; g.K = c.Kp;
     g.nb1 = c.B; g.nb2 = c.G;
-    g.row_bias = bias;  // round(round(sum) + bias[channel])
-    g.sR2 = c.Og;
+    g.bias = bias;  // round(round(sum) + bias[channel])
+    g.row_bias = bias != nullptr;
     return launch_bmm(dtype, g, kEpiPlain, true, s);
   }
 

@@ -28,10 +28,6 @@ struct BmmArgs {
   const void* B2;
   void* C;
   const void* bias;
-  // Plain epilogue, K-major B, no row groups: C row m of inner batch b2 becomes round(round(acc) + row_bias[b2*sR2 + m])
-  // (a convolution's channel bias, added after the GEMM's rounding); nullptr: none.
-  const void* row_bias;
-  int64_t sR2;
   int64_t M, N, K;
   int64_t lda, ldb, ldc;
   int64_t nb1, nb2, gB;
@@ -43,6 +39,13 @@ struct BmmArgs {
   // filled by the launcher
   int64_t tiles_m, tiles_n, total;
   int32_t a_vec, b_vec, c_vec;
+  // Plain epilogue, K-major B, no row groups: bias has one element per row of each inner batch, and C row m
+  // of inner batch b2 becomes round(round(acc) + bias[b2*M + m]) (a convolution's channel bias, added
+  // after the GEMM's rounding).
+  int32_t row_bias;
+  // N-major B: columns past N that its rows hold (a zero-padded copy has whole 16-byte chunks of columns,
+  // which the direct loads need; they reach no output).
+  int32_t b_extra;
   int32_t nt_store;  // four-wave entries: whole tiles store with non-temporal stores
 };
 

@@ -153,7 +153,7 @@ __device__ __forceinline__ void bmm_tile(const BmmArgs& args, uint32_t t, char* 
   src.p0 = reinterpret_cast<const T*>(args.B) + boff;
   src.p1 = EPI == kEpiSwiglu ? reinterpret_cast<const T*>(args.B2) + boff : src.p0;
   src.ld = args.ldb;
-  src.ncols = args.N - n0;
+  src.ncols = args.N - n0 + (BKM || GRP ? 0 : args.b_extra);
   src.swiglu = EPI == kEpiSwiglu;
   src.vec_ok = args.b_vec != 0;
   const int64_t rows = o.m_end - m0;
@@ -173,9 +173,13 @@ __device__ __forceinline__ void bmm_tile(const BmmArgs& args, uint32_t t, char* 
   }
 
   T* Cp = reinterpret_cast<T*>(args.C) + b1 * args.sC1 + b2 * args.sC2 + m0 * args.ldc + n0;
-  const T* bias = (EPI != kEpiSwiglu && args.bias) ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
-  constexpr bool kRowBias = EPI != kEpiSwiglu && BKM && !GRP;
-  const T* row_bias = (kRowBias && args.row_bias) ? reinterpret_cast<const T*>(args.row_bias) + b2 * args.sR2 + m0 : nullptr;
+  constexpr bool kRowBias = EPI == kEpiPlain && BKM && !GRP;
+  const T* bias = nullptr;
+  const T* row_bias = nullptr;
+  if (EPI != kEpiSwiglu && args.bias) {
+    if (kRowBias && args.row_bias) row_bias = reinterpret_cast<const T*>(args.bias) + b2 * args.M + m0;
+    else bias = reinterpret_cast<const T*>(args.bias) + n0;
+  }
   Tile::template epilogue<EPI == kEpiSwiglu, kRowBias>(smem, acc, Cp, args.ldc, rows < BM ? (int)rows : BM,
                                                        cols < kCols ? (int)cols : kCols, bias, row_bias,
                                                        args.c_vec != 0);
@@ -232,9 +236,9 @@ __device__ __forceinline__ void skinny_store(const BmmArgs& args, const TileOrig
   const int wr = w / S::CWC, wc = w % S::CWC;
   const int64_t n0 = o.n0 + S::WC * wc;
   T* Cp = reinterpret_cast<T*>(args.C) + o.b1 * args.sC1 + o.b2 * args.sC2 + (o.m0 + S::WR * wr) * args.ldc + n0;
-  const T* bias = args.bias ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
+  const T* bias = (args.bias && !args.row_bias) ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
   const int wrows = rows - S::WR * wr, wcols = cols - S::WC * wc;
-  const T* row_bias = args.row_bias ? reinterpret_cast<const T*>(args.row_bias) + o.b2 * args.sR2 + o.m0 + S::WR * wr : nullptr;
+  const T* row_bias = args.row_bias ? reinterpret_cast<const T*>(args.bias) + o.b2 * args.M + o.m0 + S::WR * wr : nullptr;
   S::Math::store(acc, Cp, args.ldc, wrows < S::WR ? wrows : S::WR, wcols < S::WC ? wcols : S::WC, bias, row_bias);
 }
 
@@ -294,7 +298,9 @@ void big_kernel(BmmArgs args) {
   const int rows = rows64 < BM ? (int)rows64 : BM;
   const int cols = cols64 < BN ? (int)cols64 : BN;
   typename Tile::Acc acc[Tile::FM][Tile::FN];
-  Tile::mainloop(smem, acc, A, args.lda, rows, B, args.ldb, cols, args.K);
+  const int64_t bcols64 = cols64 + args.b_extra;  // columns of B to load from (N-major)
+  const int bcols = BKM ? cols : (bcols64 < BN ? (int)bcols64 : BN);
+  Tile::mainloop(smem, acc, A, args.lda, rows, B, args.ldb, bcols, args.K);
   T* Cp = reinterpret_cast<T*>(args.C) + o.b1 * args.sC1 + o.b2 * args.sC2 + o.m0 * args.ldc + o.n0;
   const T* bias = args.bias ? reinterpret_cast<const T*>(args.bias) + o.n0 : nullptr;
   Tile::epilogue(acc, Cp, args.ldc, rows, cols, bias, args.nt_store != 0);
@@ -388,7 +394,7 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skin
   // Four-wave entries: the skinny conditions (direct loads, K-major B, plain rows, no SwiGLU),
   // or the same with a 16-bit N-major B; 32-bit output offsets inside a 256-row tile.
   // Not built for a row bias.
-  const bool big_ok = a.row_bias == nullptr && (skinny_ok || (nmajor16 && !swiglu && !grouped)) && dtype != BIOPS_F32 &&
+  const bool big_ok = a.row_bias == 0 && (skinny_ok || (nmajor16 && !swiglu && !grouped)) && dtype != BIOPS_F32 &&
                       a.ldc < (int64_t(1) << 23);
   if (forced >= kBigCfg && forced < kBigEnd && big_ok) return forced;
   // The weight-streaming entries: grouped rows, 16-bit N-major B on the direct path.
@@ -728,8 +734,8 @@ static int prepare_bmm(int dtype, BmmArgs& a, int epi, bool b_kmajor, bool& dire
   if (a.gB <= 0) a.gB = 1;
   if (a.nb2 <= 0) a.nb2 = 1;
   // Direct global->LDS loads need whole 16-byte chunks: aligned operands, K a multiple of the
-  // 128-byte step, and B K-major or N-major with N a multiple of 16 / elt.
-  direct = a.a_vec && a.b_vec && ((a.K * elt) % kKBytes == 0) && (b_kmajor || (a.N * elt) % 16 == 0) &&
+  // 128-byte step, and B K-major or N-major with whole chunks of columns.
+  direct = a.a_vec && a.b_vec && ((a.K * elt) % kKBytes == 0) && (b_kmajor || ((a.N + a.b_extra) * elt) % 16 == 0) &&
            !direct_disabled();
   // Grouped rows run on the table entries only (the skinny and large-tile kernels take a fixed
   // tile count from the host); those two read K-major B only.
@@ -974,34 +980,39 @@ extern "C" int biops_gemm(int dtype, int64_t M, int64_t N, int64_t K, const void
 }
 
 // ------------------------------------------------------------------ K padding ----
-// dst [rows_out, cols_out] = src [rows, cols] zero-extended; one 16-byte output chunk per thread
-// and iteration.  Whole chunks of a 16-byte aligned source are read with one load, others
-// element by element (a row of odd length is not 16-byte aligned after the first).
+// dst [rows_out, cols_out] = src [rows, cols] zero-extended, for up to two operands in one launch;
+// one 16-byte output chunk per thread and iteration, whole chunks with one load at any alignment.
+// I: 32-bit chunk indices where they fit (three divisions per chunk).  MI355X, both operands: 77 x
+// 3000 and 3000 x 513 fp32 12.3 -> 9.5 us (two launches, 64-bit indices, element-wise loads of
+// misaligned rows before), 100 x 1367 and 3096 x 1367 bf16 14.9 -> 9.9 us.
 struct PadArgs {
   const void* src;
   void* dst;
   int64_t rows, cols, ld, rows_out, cols_out;
   int64_t batches, sbatch;  // source matrices and their stride (elements); destinations follow each other
-  int32_t vec;              // src, ld and sbatch 16-byte aligned
+};
+struct PadPair {
+  PadArgs op[2];
+  int64_t first, total;  // chunks of op[0], of both
 };
 
-template <int E>
-__global__ __launch_bounds__(256) void pad_rows_kernel(PadArgs a) {
+template <int E, typename I>
+__global__ __launch_bounds__(256) void pad_rows_kernel(PadPair p) {
   using W = typename std::conditional<E == 2, uint16_t, uint32_t>::type;
   constexpr int V = 16 / E;
-  const int64_t cpr = a.cols_out / V;
-  const int64_t per = a.rows_out * cpr;  // chunks of one destination matrix
-  const int64_t total = a.batches * per;
-  const W* src = reinterpret_cast<const W*>(a.src);
-  W* dst = reinterpret_cast<W*>(a.dst);
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t b = i / per, j = i - b * per;
-    const int64_t r = j / cpr, k0 = (j - r * cpr) * V;
+  for (I g = (I)blockIdx.x * 256 + threadIdx.x; g < (I)p.total; g += (I)gridDim.x * 256) {
+    const bool second = g >= (I)p.first;
+    const PadArgs& a = p.op[second ? 1 : 0];
+    const I i = second ? g - (I)p.first : g;
+    const I cpr = (I)(a.cols_out / V), per = (I)a.rows_out * cpr;  // chunks of a row, of one destination matrix
+    const I b = i / per, j = i - b * per;
+    const I r = j / cpr;
+    const int64_t k0 = (int64_t)(j - r * cpr) * V;
     u32x4_t v = {0u, 0u, 0u, 0u};
-    if (r < a.rows && k0 < a.cols) {
-      const W* s = src + b * a.sbatch + r * a.ld + k0;
-      if (a.vec && k0 + V <= a.cols) {
-        v = *reinterpret_cast<const u32x4_t*>(s);
+    if ((int64_t)r < a.rows && k0 < a.cols) {
+      const W* s = reinterpret_cast<const W*>(a.src) + (int64_t)b * a.sbatch + (int64_t)r * a.ld + k0;
+      if (k0 + V <= a.cols) {
+        v = load_16(s);
       } else {
         W e[V];
 #pragma unroll
@@ -1009,36 +1020,57 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(PadArgs a) {
         v = __builtin_bit_cast(u32x4_t, e);
       }
     }
-    *reinterpret_cast<u32x4_t*>(dst + i * V) = v;
+    *reinterpret_cast<u32x4_t*>(reinterpret_cast<W*>(a.dst) + (int64_t)i * V) = v;
   }
 }
 
-static int pad_rows(int dtype, int64_t rows, int64_t cols, const void* src, int64_t ld_src, int64_t rows_out,
-                    int64_t cols_out, void* dst, hipStream_t stream, int64_t batches = 1, int64_t sbatch = 0) {
+// The operands with rows_out and cols_out > 0 of `n` (at most two).
+static int pad_rows(int dtype, const PadArgs* ops, int n, hipStream_t stream) {
   const int elt = dtype_bytes(dtype);
   if (!is_float_dtype(dtype)) return fail(BIOPS_ERR_DTYPE, "unsupported dtype %d", dtype);
-  if (rows < 0 || cols < 0 || rows_out < rows || cols_out < cols)
-    return fail(BIOPS_ERR_ARG, "padded shape [%lld, %lld] smaller than [%lld, %lld]", (long long)rows_out,
-                (long long)cols_out, (long long)rows, (long long)cols);
-  if ((cols_out * elt) % 16 != 0 || reinterpret_cast<uintptr_t>(dst) % 16 != 0)
-    return fail(BIOPS_ERR_LAYOUT, "padded rows must be whole 16-byte chunks on a 16-byte aligned base");
-  if (rows > 1 && ld_src < cols) return fail(BIOPS_ERR_LAYOUT, "source rows overlap");
-  if (rows_out == 0 || cols_out == 0) return BIOPS_OK;
-  if (!dst || (rows > 0 && cols > 0 && !src)) return fail(BIOPS_ERR_ARG, "null operand");
-  PadArgs a{src, dst, rows, cols, ld_src, rows_out, cols_out, batches, sbatch, 0};
-  a.vec = reinterpret_cast<uintptr_t>(src) % 16 == 0 && (ld_src * elt) % 16 == 0 && (sbatch * elt) % 16 == 0;
-  const int64_t chunks = batches * rows_out * (cols_out * elt / 16);
-  const int64_t blocks = std::min<int64_t>(cdiv(chunks, 256), 8192);
-  if (elt == 2)
-    hipLaunchKernelGGL(pad_rows_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
-  else
-    hipLaunchKernelGGL(pad_rows_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  PadPair p{};
+  int used = 0;
+  for (int i = 0; i < n; ++i) {
+    const PadArgs& a = ops[i];
+    if (a.rows < 0 || a.cols < 0 || a.rows_out < a.rows || a.cols_out < a.cols)
+      return fail(BIOPS_ERR_ARG, "padded shape [%lld, %lld] smaller than [%lld, %lld]", (long long)a.rows_out,
+                  (long long)a.cols_out, (long long)a.rows, (long long)a.cols);
+    if ((a.cols_out * elt) % 16 != 0 || reinterpret_cast<uintptr_t>(a.dst) % 16 != 0)
+      return fail(BIOPS_ERR_LAYOUT, "padded rows must be whole 16-byte chunks on a 16-byte aligned base");
+    if (a.rows > 1 && a.ld < a.cols) return fail(BIOPS_ERR_LAYOUT, "source rows overlap");
+    if (a.rows_out == 0 || a.cols_out == 0) continue;
+    if (!a.dst || (a.rows > 0 && a.cols > 0 && !a.src)) return fail(BIOPS_ERR_ARG, "null operand");
+    p.op[used++] = a;
+    const int64_t chunks = a.batches * a.rows_out * (a.cols_out * elt / 16);
+    if (used == 1) p.first = chunks;
+    p.total += chunks;
+  }
+  if (p.total == 0) return BIOPS_OK;
+  const int64_t blocks = std::min<int64_t>(cdiv(p.total, 256), 8192);
+  const dim3 grid((unsigned)blocks);
+  const bool small = p.total < (int64_t(1) << 32) - (int64_t(1) << 22);  // room for one more grid stride
+  if (elt == 2) {
+    if (small) hipLaunchKernelGGL((pad_rows_kernel<2, uint32_t>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((pad_rows_kernel<2, int64_t>), grid, dim3(256), 0, stream, p);
+  } else {
+    if (small) hipLaunchKernelGGL((pad_rows_kernel<4, uint32_t>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((pad_rows_kernel<4, int64_t>), grid, dim3(256), 0, stream, p);
+  }
   return check_launch("pad_rows_kernel");
+}
+
+// Operands the direct loads can read as they are: 16-byte aligned, non-overlapping rows, and K
+// (rows of it K-major, that many rows N-major) a whole number of 128-byte steps, N-major with whole
+// 16-byte chunks of columns.
+static bool whole_steps(const PadArgs& a, int64_t K, bool kmajor, int elt) {
+  return reinterpret_cast<uintptr_t>(a.src) % 16 == 0 && (a.ld * elt) % 16 == 0 && (a.sbatch * elt) % 16 == 0 &&
+         a.ld >= a.cols && (K * elt) % kKBytes == 0 && (kmajor || (a.cols * elt) % 16 == 0);
 }
 
 extern "C" int biops_pad_rows(int dtype, int64_t rows, int64_t cols, const void* src, int64_t ld_src,
                               int64_t rows_out, int64_t cols_out, void* dst, void* stream) {
-  return pad_rows(dtype, rows, cols, src, ld_src, rows_out, cols_out, dst, (hipStream_t)stream);
+  const PadArgs a{src, dst, rows, cols, ld_src, rows_out, cols_out, 1, 0};
+  return pad_rows(dtype, &a, 1, (hipStream_t)stream);
 }
 
 // Padded operands of biops_gemm_padded: A [M, Kp] at the workspace base, B [N, Kp] (K-major) or
@@ -1087,14 +1119,19 @@ extern "C" int biops_gemm_padded(int dtype, int64_t M, int64_t N, int64_t K, con
   char* ap = static_cast<char*>(workspace);
   char* bp = ap + p.a_bytes;
   const hipStream_t s = (hipStream_t)stream;
-  int rc = pad_rows(dtype, M, K, A, sAm, M, p.kp, ap, s);
-  if (rc != BIOPS_OK) return rc;
-  rc = kmajor ? pad_rows(dtype, N, K, B, ldb, N, p.kp, bp, s) : pad_rows(dtype, K, N, B, ldb, p.kp, p.np, bp, s);
+  // an operand that needs no padding is read in place
+  PadArgs ops[2] = {PadArgs{A, ap, M, K, sAm, M, p.kp, 1, 0},
+                    kmajor ? PadArgs{B, bp, N, K, ldb, N, p.kp, 1, 0} : PadArgs{B, bp, K, N, ldb, p.kp, p.np, 1, 0}};
+  const bool a_ok = whole_steps(ops[0], K, true, elt), b_ok = whole_steps(ops[1], K, kmajor, elt);
+  const int n = a_ok && b_ok ? 0 : (a_ok || b_ok ? 1 : 2);
+  if (a_ok) ops[0] = ops[1];
+  const int rc = pad_rows(dtype, ops, n, s);
   if (rc != BIOPS_OK) return rc;
   BmmArgs a{};
-  a.A = ap; a.B = bp; a.B2 = nullptr; a.C = C; a.bias = bias;
+  a.A = a_ok ? A : ap; a.B = b_ok ? B : bp; a.B2 = nullptr; a.C = C; a.bias = bias;
   a.M = M; a.N = N; a.K = p.kp;
-  a.lda = p.kp; a.ldb = kmajor ? p.kp : p.np; a.ldc = sCm;
+  a.lda = a_ok ? sAm : p.kp; a.ldb = b_ok ? ldb : (kmajor ? p.kp : p.np); a.ldc = sCm;
+  a.b_extra = (int32_t)(p.np - N);
   a.nb1 = 1; a.nb2 = 1; a.gB = 1;
   return launch_bmm(dtype, a, bias ? kEpiBias : kEpiPlain, kmajor, s);
 }
@@ -1139,17 +1176,21 @@ extern "C" int biops_bmm_padded(int dtype, int64_t batch, int64_t M, int64_t N, 
   char* ap = static_cast<char*>(workspace);
   char* bp = ap + p.a_bytes;
   const hipStream_t s = (hipStream_t)stream;
-  int rc = pad_rows(dtype, M, K, A, sAm, M, p.kp, ap, s, na, sA);
-  if (rc != BIOPS_OK) return rc;
-  rc = kmajor ? pad_rows(dtype, N, K, B, ldb, N, p.kp, bp, s, nb, sB) : pad_rows(dtype, K, N, B, ldb, p.kp, p.np, bp, s, nb, sB);
+  PadArgs ops[2] = {PadArgs{A, ap, M, K, sAm, M, p.kp, na, sA},
+                    kmajor ? PadArgs{B, bp, N, K, ldb, N, p.kp, nb, sB} : PadArgs{B, bp, K, N, ldb, p.kp, p.np, nb, sB}};
+  const bool a_ok = whole_steps(ops[0], K, true, elt), b_ok = whole_steps(ops[1], K, kmajor, elt);
+  const int n = a_ok && b_ok ? 0 : (a_ok || b_ok ? 1 : 2);
+  if (a_ok) ops[0] = ops[1];
+  const int rc = pad_rows(dtype, ops, n, s);
   if (rc != BIOPS_OK) return rc;
   BmmArgs a{};
-  a.A = ap; a.B = bp; a.B2 = nullptr; a.C = C; a.bias = nullptr;
+  a.A = a_ok ? A : ap; a.B = b_ok ? B : bp; a.B2 = nullptr; a.C = C; a.bias = nullptr;
   a.M = M; a.N = N; a.K = p.kp;
-  a.lda = p.kp; a.ldb = kmajor ? p.kp : p.np; a.ldc = sCm;
+  a.lda = a_ok ? sAm : p.kp; a.ldb = b_ok ? ldb : (kmajor ? p.kp : p.np); a.ldc = sCm;
+  a.b_extra = (int32_t)(p.np - N);
   a.nb1 = batch; a.nb2 = 1; a.gB = 1;
-  a.sA1 = na == 1 ? 0 : M * p.kp;
-  a.sB1 = nb == 1 ? 0 : (kmajor ? N * p.kp : p.kp * p.np);
+  a.sA1 = a_ok ? sA : (na == 1 ? 0 : M * p.kp);
+  a.sB1 = b_ok ? sB : (nb == 1 ? 0 : (kmajor ? N * p.kp : p.kp * p.np));
   a.sC1 = sC;
   return launch_bmm(dtype, a, kEpiPlain, kmajor, s);
 }

@@ -32,14 +32,6 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// 16 bytes at any element boundary: rows of an odd length start anywhere.  The GPU takes 16-byte
-// global loads and stores at any alignment (one more 64-byte segment per wavefront access), so
-// misaligned rows need no element-wise path.
-typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));
-typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
-
-__device__ __forceinline__ u32x4_t load_16(const void* p) { return *reinterpret_cast<const u32x4_any_t*>(p); }
-
 template <typename T>
 __device__ __forceinline__ void unpack_chunk(const u32x4_t& raw, float (&v)[16 / sizeof(T)]) {
   if constexpr (sizeof(T) == 4) {

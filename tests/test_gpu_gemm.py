@@ -529,3 +529,33 @@ def test_bmm_padded_k_gives_the_register_path_bits(monkeypatch, dtype, batch, m,
     assert_bitwise(bmm_persistent(a[1:2], b[1:2]), reg[1:2], "one batch element")
     ref = oracle.bmm(a_cpu.contiguous(), b_cpu)
     assert_gemm_close(padded, ref, a_cpu.double().abs() @ b_cpu.double().abs(), k)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch", (0, 3))
+@pytest.mark.parametrize(("a_cut", "n", "layout"), (
+    (1, 96, "cols"),   # only A misaligned: a K-major B is read in place
+    (1, 96, "rows"),   # the same with a row-major B
+    (0, 97, "rows"),   # only B padded (N not whole 16-byte chunks), A in place
+    (0, 131, "rows"),  # and a last tile of three columns
+    (1, 5, "rows"),    # both copied, fewer columns than a chunk
+))
+def test_padding_copies_only_the_operand_that_needs_it(monkeypatch, dtype, batch, a_cut, n, layout):
+    """K is a whole number of 128-byte steps: an aligned operand of a padded product is read where
+    it is, a row-major B of any N has its padded columns read and never stored, and the bits are
+    the register path's."""
+    import batch_invariant_ops.batch_invariant_ops as bio
+
+    m, k, nb = 67, 256, max(batch, 1)
+    a = gpu(randn(nb, m, k + a_cut, seed=5900 + n, dtype=dtype))[:, :, a_cut:]
+    b = gpu(randn(nb, k, n, seed=5901 + n, dtype=dtype) * 0.05)
+    if layout == "cols":
+        b = b.transpose(1, 2).contiguous().transpose(1, 2)
+    run = bmm_persistent if batch else (lambda x, y: matmul_persistent(x[0], y[0]))
+    monkeypatch.setattr(bio, "_PAD_MIN_WORK", 1 << 62)
+    reg = run(a, b)
+    monkeypatch.setattr(bio, "_PAD_MIN_WORK", 0)
+    monkeypatch.setattr(bio, "_PAD_MIN_K_BYTES", 0)
+    monkeypatch.setattr(bio, "_PAD_MIN_MISALIGNED_K_BYTES", 0)
+    assert bio._padded_workspace(a if batch else a[0], b if batch else b[0], m, n, k, batch) > 0
+    assert_bitwise(run(a, b), reg, "padded vs register path")
