@@ -78,6 +78,14 @@ _SIGNATURES = {
         + [_p, _l, _l, _l] * 3
         + [_p, _i, _l, _l, _l, _l, _f, _p, _p, _l, _p],
     ),
+    "biops_sdpa_f32_supported": (_i, [_l, _l, _l, _l, _l, _l]),
+    "biops_sdpa_f32_workspace_size": (_l, [_l, _l, _l, _l, _l, _l]),
+    "biops_sdpa_f32": (
+        _i,
+        [_l, _l, _l, _l, _l, _l, _l]
+        + [_p, _l, _l, _l] * 3
+        + [_p, _i, _l, _l, _l, _l, _i, _f, _p, _p, _l, _p],
+    ),
     "biops_varlen_sdpa_fused": (
         _i,
         [_i, _l, _l, _l, _l] + [_p, _l, _l] * 4 + [_p, _p, _p, _i, _f, _p],
@@ -193,7 +201,7 @@ def function(name: str):
 # same C functions and arguments, without ctypes' per-argument conversions.
 _FAST = {"biops_gemm": "gemm", "biops_gemm_padded": "gemm_padded", "biops_reduce": "reduce", "biops_softmax": "softmax",
          "biops_sdpa_fused": "sdpa_fused", "biops_sdpa_split": "sdpa_split",
-         "biops_sdpa_split_workspace_size": "sdpa_split_workspace_size",
+         "biops_sdpa_split_workspace_size": "sdpa_split_workspace_size", "biops_sdpa_f32": "sdpa_f32",
          "biops_varlen_plan": "varlen_plan", "biops_varlen_fused_order": "varlen_fused_order",
          "biops_varlen_sdpa_fused": "varlen_sdpa_fused",
          "biops_varlen_sdpa_fused_planned": "varlen_sdpa_fused_planned"}

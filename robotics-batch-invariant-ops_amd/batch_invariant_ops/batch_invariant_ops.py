@@ -598,6 +598,17 @@ def _fused_attention_ok(dtype, d, dv, *tensors, varlen=False):
     return True
 
 
+def _f32_attention_ok(B, Hq, Lq, Lk, D, Dv, *tensors):
+    """True when the one-pass float32 kernel takes this call (head sizes multiples of 4 up to 128,
+    16-byte aligned rows); ``BIOPS_ATTENTION_MATERIALIZE=1`` selects the materialised path."""
+    if not nat.load().biops_sdpa_f32_supported(B, Hq, Lq, Lk, D, Dv):
+        return False
+    if nat.env_flag("BIOPS_ATTENTION_MATERIALIZE", False):
+        return False
+    return not any(t.data_ptr() % 16 or t.stride(2) >= 1 << 25 or any(st % 4 for st in t.stride()[:-1])
+                   for t in tensors)
+
+
 def _sdpa_glue(q4, k4, v4, group, mask4, scale, out_dtype):
     """Eager SDPA for mask dtypes the fused softmax does not take (type promotion): the GEMMs
     and the softmax are the library kernels, the masking is the reference's elementwise glue
@@ -726,6 +737,21 @@ def scaled_dot_product_attention_batch_invariant(
             causal_code, float(scale_value), out.data_ptr(), nat.stream_of(out),
         )
         nat.check(rc, "biops_sdpa_fused")
+        return out.reshape(*leading, Lq, Dv)
+    if query.dtype == torch.float32 and _f32_attention_ok(B, Hq, Lq, Lk, D, Dv, q4, k4, v4):
+        ws_bytes = nat.load().biops_sdpa_f32_workspace_size(B, Hq, Lq, Lk, D, Dv)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
+        rc = _fast_fn("biops_sdpa_f32")(
+            B, Hq, Hkv, Lq, Lk, D, Dv,
+            q4.data_ptr(), q4.stride(0), q4.stride(1), q4.stride(2),
+            k4.data_ptr(), k4.stride(0), k4.stride(1), k4.stride(2),
+            v4.data_ptr(), v4.stride(0), v4.stride(1), v4.stride(2),
+            mask4.data_ptr() if mask4 is not None else None, mask_code,
+            *(mask4.stride() if mask4 is not None else (0, 0, 0, 0)),
+            causal_code, float(scale_value), out.data_ptr(),
+            workspace.data_ptr() if ws_bytes else None, ws_bytes, nat.stream_of(out),
+        )
+        nat.check(rc, "biops_sdpa_f32")
         return out.reshape(*leading, Lq, Dv)
     ws_bytes = nat.load().biops_sdpa_workspace_size(nat.dtype_code(query.dtype), B, Hq, Lq, Lk)
     workspace = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=query.device)

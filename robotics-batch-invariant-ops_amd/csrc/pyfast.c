@@ -202,6 +202,21 @@ static PyObject* fast_sdpa_split(PyObject* self, PyObject* const* args, Py_ssize
   return PyLong_FromLong(rc);
 }
 
+/* sdpa_f32(batch, hq, hkv, lq, lk, d, dv, q, sqB, sqH, sqL, k, skB, skH, skL, v, svB, svH, svL, mask,
+ *          mask_dtype, mB, mH, mI, mJ, causal, scale, out, workspace, bytes, stream) */
+static PyObject* fast_sdpa_f32(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  int64_t iv[31];
+  void* pv[31];
+  float fv[31];
+  (void)self;
+  if (!parse(args, nargs, "lllllllplllplllplllpllllllfpplp", iv, pv, fv)) return NULL;
+  int rc;
+  WITHOUT_GIL(rc, biops_sdpa_f32(iv[0], iv[1], iv[2], iv[3], iv[4], iv[5], iv[6], pv[7], iv[8], iv[9], iv[10], pv[11],
+                                 iv[12], iv[13], iv[14], pv[15], iv[16], iv[17], iv[18], pv[19], (int)iv[20], iv[21],
+                                 iv[22], iv[23], iv[24], (int)iv[25], fv[26], pv[27], pv[28], iv[29], pv[30]));
+  return PyLong_FromLong(rc);
+}
+
 /* sdpa_split_workspace_size(dtype, batch, hq, hkv, lq, lk, d, dv, causal) -> bytes or -1 */
 static PyObject* fast_sdpa_split_workspace_size(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   int64_t iv[9];
@@ -252,6 +267,7 @@ static PyMethodDef kMethods[] = {
     {"varlen_fused_order", (PyCFunction)(void (*)(void))fast_varlen_fused_order, METH_FASTCALL,
      "biops_varlen_fused_order"},
     {"sdpa_split", (PyCFunction)(void (*)(void))fast_sdpa_split, METH_FASTCALL, "biops_sdpa_split"},
+    {"sdpa_f32", (PyCFunction)(void (*)(void))fast_sdpa_f32, METH_FASTCALL, "biops_sdpa_f32"},
     {"sdpa_split_workspace_size", (PyCFunction)(void (*)(void))fast_sdpa_split_workspace_size, METH_FASTCALL,
      "biops_sdpa_split_workspace_size"},
     {"varlen_sdpa_fused", (PyCFunction)(void (*)(void))fast_varlen_sdpa_fused, METH_FASTCALL,

@@ -1,0 +1,128 @@
+"""One-pass float32 attention: parity with the CPU oracle and with the materialised path, masks in
+every layout, bitwise batch invariance.
+
+Tolerance (tests/_parity.py, as for the materialised float32 path): rtol 1e-5 of |O| + 2 (P |V|) per
+element.  The kernel's own error is some 2^-24 times the root of the longest sum (head size and
+key count below 2^10 here), well inside it.
+"""
+
+import math
+
+import pytest
+import torch
+
+from batch_invariant_ops import scaled_dot_product_attention_batch_invariant as sdpa
+from batch_invariant_ops import _native as nat
+
+from _parity import check_sdpa
+from _tol import assert_bitwise
+
+
+def randn(*shape, seed):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
+
+
+def test_sizes_taken_and_argument_errors():
+    lib = nat.load(require_gpu=False)
+    ok = lib.biops_sdpa_f32_supported
+    assert ok(2, 4, 7, 9, 4, 128) and ok(1, 1, 1, 0, 128, 4)
+    assert not ok(1, 1, 1, 1, 132, 4) and not ok(1, 1, 1, 1, 6, 4) and not ok(1, 1, 1, 1, 4, 130)
+    p = 256
+
+    def call(d=64, q=p, sk=64, hkv=2, mask=None, mcode=0, causal=0):
+        return lib.biops_sdpa_f32(1, 4, hkv, 3, 5, d, 64, q, 0, 0, 64, p, 0, 0, sk, p, 0, 0, 64, mask, mcode, 0, 0, 5, 1,
+                                  causal, 1.0, p, None, 0, None)
+
+    assert call(d=66) == 5 and call(hkv=3) == 1 and call(q=None) == 1
+    assert call(q=p + 4) == 2 and call(sk=66) == 2
+    assert call(mask=p, mcode=nat.BF16) == 3 and call(mask=p, mcode=nat.BOOL, causal=1) == 1
+
+
+SHAPES = (
+    # B, Hq, Hkv, Lq, Lk, D, Dv: query rows around the 128-row tile and its 32-row wavefronts, keys around
+    # the 32-key block, head sizes on both sides of every class of the dispatch
+    (2, 4, 2, 129, 257, 64, 64),
+    (1, 2, 1, 128, 33, 72, 72),
+    (2, 3, 3, 31, 32, 68, 96),
+    (1, 2, 2, 33, 31, 80, 40),
+    (1, 2, 2, 1, 1, 4, 4),
+    (1, 4, 1, 200, 95, 96, 8),
+    (1, 2, 2, 161, 300, 128, 128),
+    (2, 2, 1, 97, 64, 100, 64),
+    (1, 1, 1, 5, 65, 8, 100),
+)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ("full", "causal", "boolean", "additive"))
+@pytest.mark.parametrize("shape", SHAPES)
+def test_f32_sdpa_matches_oracle_and_materialized(shape, kind, monkeypatch):
+    B, Hq, Hkv, Lq, Lk, D, Dv = shape
+    seed = 9500 + 10 * SHAPES.index(shape)
+    q, k, v = randn(B, Hq, Lq, D, seed=seed), randn(B, Hkv, Lk, D, seed=seed + 1), randn(B, Hkv, Lk, Dv, seed=seed + 2)
+    kw = dict(enable_gqa=Hq != Hkv, is_causal=kind == "causal")
+    mask = None
+    if kind in ("boolean", "additive"):
+        keep = torch.rand(B, 1, Lq, Lk, generator=torch.Generator().manual_seed(seed + 3)) > 0.3
+        keep[:, :, Lq // 2] = False  # a fully masked row gives 0
+        keep[:, :, :, : Lk // 2] &= torch.arange(Lq).view(-1, 1) % 2 == 0  # the maximum appears late
+        mask = keep
+        if kind == "additive":
+            mask = torch.rand(B, 1, Lq, Lk, generator=torch.Generator().manual_seed(seed + 4)) * -10
+            mask[~keep] = -math.inf
+    dev = dict(kw, attn_mask=None if mask is None else mask.cuda())
+    out = sdpa(q.cuda(), k.cuda(), v.cuda(), **dev)
+    check_sdpa(out, q, k, v, attn_mask=mask, what=f"float32 vs oracle {shape}", **kw)
+    if mask is not None:
+        assert torch.count_nonzero(out[:, :, Lq // 2]) == 0
+        wide = torch.zeros(B, 1, Lq, 2 * Lk + 3, dtype=mask.dtype)  # same mask, key stride 2, odd row stride
+        wide[..., 1:1 + 2 * Lk:2] = mask
+        strided = sdpa(q.cuda(), k.cuda(), v.cuda(), **dict(kw, attn_mask=wide.cuda()[..., 1:1 + 2 * Lk:2]))
+        assert_bitwise(strided, out, "strided mask")
+    monkeypatch.setenv("BIOPS_ATTENTION_MATERIALIZE", "1")
+    mat = sdpa(q.cuda(), k.cuda(), v.cuda(), **dev)
+    assert torch.allclose(out, mat, rtol=1e-5, atol=2e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ("full", "causal", "boolean"))
+@pytest.mark.parametrize("D", (64, 72, 128))
+def test_f32_sdpa_is_batch_invariant(D, kind):
+    """Samples alone (a workgroup per 128 keys), a batch that fills the chip (the workgroups merge their
+    keys themselves), and views of wider buffers (head and row strides of their own)."""
+    B, Lk = 48, 290
+    assert nat.load().biops_sdpa_f32_workspace_size(1, 6, 150, Lk, D, D) > 0
+    assert nat.load().biops_sdpa_f32_workspace_size(B, 6, 150, Lk, D, D) == 0
+    q = randn(B, 150, 6, D, seed=9700).cuda().transpose(1, 2)
+    kc, vc = (randn(B, 310, 2, D + 4, seed=9701 + i).cuda() for i in range(2))
+    k, v = (x[:, 9:9 + Lk, :, :D].transpose(1, 2) for x in (kc, vc))
+    mask = None
+    if kind == "boolean":
+        mask = torch.rand(B, 1, 150, Lk, generator=torch.Generator().manual_seed(9710)) > 0.3
+        mask[:, :, ::3, :128] = False  # a whole group of keys masked out
+        mask[:, :, 7] = False
+        mask = mask.cuda()
+
+    def run(sl, contiguous=False):
+        args = [x[sl].contiguous() if contiguous else x[sl] for x in (q, k, v)]
+        return sdpa(*args, attn_mask=None if mask is None else mask[sl], is_causal=kind == "causal", enable_gqa=True)
+
+    full = run(slice(0, B))
+    for j in (0, 21, 47):
+        one = slice(j, j + 1)
+        assert_bitwise(run(one), full[one], f"sample {j}")
+        assert_bitwise(run(one, contiguous=True), full[one], f"sample {j} contiguous")
+
+
+@pytest.mark.gpu
+def test_f32_sdpa_large_scores_and_unread_rows():
+    """Scores of several hundred (the running maximum grows block by block), NaN past the keys."""
+    q = randn(1, 2, 70, 64, seed=9800)
+    k = randn(1, 2, 130, 64, seed=9801) * torch.linspace(1, 30, 130).view(1, 1, -1, 1)
+    v = randn(1, 2, 130, 64, seed=9802)
+    kc, vc = (torch.full((1, 2, 200, 64), math.nan, device="cuda") for _ in "kv")
+    kc[:, :, :130], vc[:, :, :130] = k.cuda(), v.cuda()
+    out = sdpa(q.cuda(), kc[:, :, :130], vc[:, :, :130])
+    # the scores' own rounding (relative 2^-24 of up to 2^10) moves a probability by up to 2^-13
+    ref = torch.softmax((q.double() @ k.double().transpose(-1, -2)) / 8.0, -1) @ v.double()
+    assert torch.allclose(out.cpu().double(), ref, rtol=2.0**-11, atol=2.0**-11)
