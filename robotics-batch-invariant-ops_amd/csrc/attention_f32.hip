@@ -59,13 +59,21 @@ struct F32AttnArgs {
   float* stats;
 };
 
+// exp(x - m).  The difference is taken before the factor log2 e: a row of which every key carries a
+// mask of the type's lowest value has a finite maximum whose multiple by log2 e is not (fma(x, log2 e,
+// -m log2 e) gave NaN there).
+__device__ __forceinline__ float f32_exp(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * kLog2e); }
+
+// False for a chunk without a visible key.  A chunk whose scores are all NaN has the maximum -inf too,
+// but a NaN sum.
+__device__ __forceinline__ bool f32_any(float m, float l) { return m != -INFINITY || l != 0.f; }
+
 // Adds a chunk's (mc, lc) with at least one visible key to the running (m, l); the running O becomes
 // O * c1 + Oc * c2 (f32_merge_o).
 __device__ __forceinline__ void f32_merge(float& m, float& l, float mc, float lc, float& c1, float& c2) {
   const float mn = fmaxf(m, mc);
-  const float sh = mn * kLog2e;
-  c1 = m == mn ? 1.f : __builtin_amdgcn_exp2f(__builtin_fmaf(m, kLog2e, -sh));
-  c2 = mc == mn ? 1.f : __builtin_amdgcn_exp2f(__builtin_fmaf(mc, kLog2e, -sh));
+  c1 = m == mn ? 1.f : f32_exp(m, mn);
+  c2 = mc == mn ? 1.f : f32_exp(mc, mn);
   l = __builtin_fmaf(l, c1, lc * c2);
   m = mn;
 }
@@ -73,7 +81,7 @@ __device__ __forceinline__ float f32_merge_o(float o, float oc, float c1, float 
   const float t = oc * c2;
   return first ? t : __builtin_fmaf(o, c1, t);
 }
-__device__ __forceinline__ float f32_inverse(float m, float l) { return m == -INFINITY || l == 0.f ? 0.f : 1.0f / l; }
+__device__ __forceinline__ float f32_inverse(float l) { return l == 0.f ? 0.f : 1.0f / l; }
 
 // MASK: 0 none, 1 boolean (bytes, nonzero = keep), 2 additive.  DP, DVP: head and value size rounded up
 // to 32 elements; QP: chunk pairs (8 elements) of the head size that are multiplied (zeros beyond).
@@ -257,10 +265,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
     else transform(std::false_type{});
     bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
     const float mn = fmaxf(m, bm);
-    const float sh = (mn == -INFINITY ? 0.f : mn) * kLog2e;
+    const float base = mn == -INFINITY ? 0.f : mn;
     if (__any(mn > m)) {  // some row's maximum grew: rescale what was summed so far
-      const float c = __builtin_amdgcn_exp2f(__builtin_fmaf(m, kLog2e, -sh));
-      // a row whose maximum stayed keeps its sums exactly (its c is 2^rounding, not 1)
+      const float c = f32_exp(m, base);
       const float cc = mn > m ? c : 1.f;
       l *= cc;
 #pragma unroll
@@ -272,7 +279,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
     float part = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      acc[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[r], kLog2e, -sh));
+      acc[r] = f32_exp(acc[r], base);
       part += acc[r];
     }
     l += part;
@@ -309,11 +316,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
       return;
     }
     // the last chunk's merge divides by the row sum and stores the result
-    const bool first = mt == -INFINITY, some = m != -INFINITY;
+    const bool first = mt == -INFINITY, some = f32_any(m, lc);
     if (row_ok && (some || last)) {
       float c1 = 1.f, c2 = 0.f;
       if (some) f32_merge(mt, lt, m, lc, c1, c2);
-      const float inv = last ? f32_inverse(mt, lt) : 1.f;
+      const float inv = last ? f32_inverse(lt) : 1.f;
 #pragma unroll
       for (int e = 0; e < OF; ++e) {
         f32x4_t o[4];  // a column block's loads before their first use (columns past dv read column 0)
@@ -379,14 +386,14 @@ __global__ __launch_bounds__(256) void f32_combine_kernel(F32AttnArgs a) {
   for (int c = 0; c < nc; ++c) {
     const f32x2_t st = *reinterpret_cast<const f32x2_t*>(a.stats + 2 * (c * rows + r));
     const f32x4_t oc = *reinterpret_cast<const f32x4_t*>(a.partial + (c * rows + r) * a.dv + col);
-    if (st[0] == -INFINITY) continue;
+    if (!f32_any(st[0], st[1])) continue;
     const bool first = m == -INFINITY;
     float c1, c2;
     f32_merge(m, l, st[0], st[1], c1, c2);
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = f32_merge_o(o[e], oc[e], c1, c2, first);
   }
-  *reinterpret_cast<f32x4_t*>(a.out + r * a.dv + col) = o * f32_inverse(m, l);
+  *reinterpret_cast<f32x4_t*>(a.out + r * a.dv + col) = o * f32_inverse(l);
 }
 
 template <int DP, int QP, int DVP, bool SPLIT>

@@ -126,3 +126,34 @@ def test_f32_sdpa_large_scores_and_unread_rows():
     # the scores' own rounding (relative 2^-24 of up to 2^10) moves a probability by up to 2^-13
     ref = torch.softmax((q.double() @ k.double().transpose(-1, -2)) / 8.0, -1) @ v.double()
     assert torch.allclose(out.cpu().double(), ref, rtol=2.0**-11, atol=2.0**-11)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", (1, 160))
+def test_f32_sdpa_masks_of_the_lowest_value(B):
+    """Padding written as the type's lowest value instead of -inf: keys in front, keys at the back, a whole
+    row (which averages V), with one workgroup per 128 keys and with one per query tile."""
+    L = 300
+    q, k, v = (randn(B, 4, L, 64, seed=9810 + i) for i in range(3))
+    mask = torch.zeros(B, 1, L, L)
+    low = torch.finfo(torch.float32).min
+    mask[:, :, 0:90, :140] = low
+    mask[:, :, 90:200, 100:] = low
+    mask[:, :, 200:210] = low
+    out = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=mask.cuda())
+    one = slice(B - 1, B)
+    check_sdpa(out[one], q[one], k[one], v[one], attn_mask=mask[one], what="lowest value")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", (1, 160))
+def test_f32_sdpa_passes_nan_on(B):
+    """A query of NaN gives NaN, also where no score of its row compares; so do 128 keys of NaN (whose
+    running maximum stays -inf) before or after others, for every row of their head."""
+    q, k, v = (randn(B, 4, 300, 64, seed=9820 + i).cuda() for i in range(3))
+    q[:, 0, 5] = math.nan
+    k[:, 1, :128] = math.nan
+    k[:, 2, 128:256] = math.nan
+    out = sdpa(q, k, v)
+    assert out[:, 0, 5].isnan().all() and out[:, 1:3].isnan().all()
+    assert out[:, 0, :5].isfinite().all() and out[:, 3].isfinite().all()
