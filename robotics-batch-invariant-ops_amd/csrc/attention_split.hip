@@ -76,6 +76,11 @@ __device__ __forceinline__ uint32_t split_pack2(float x, float y) {
   else return (uint32_t)Num<T>::to_bits(x) | ((uint32_t)Num<T>::to_bits(y) << 16);
 }
 
+// exp(x - m).  The difference is taken before the factor log2 e: keys that carry a mask of the type's
+// lowest value leave a finite maximum whose multiple by log2 e is not (a wavefront's 64 keys masked
+// that way gave NaN with fma(x, log2 e, -m log2 e)).
+__device__ __forceinline__ float split_exp(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * kLog2e); }
+
 // Workgroup barrier that waits for LDS operations only (__syncthreads also drains the global
 // loads in flight).
 __device__ __forceinline__ void lds_barrier() {
@@ -182,11 +187,11 @@ __global__ __launch_bounds__(256) void split_score_kernel(SplitArgs a) {
         else transform(std::false_type{});
       }
       m = fmaxf(m, __shfl_xor(m, 32, 64));
-      const float sh = (m == -INFINITY ? 0.f : m) * kLog2e;
+      const float base = m == -INFINITY ? 0.f : m;
 #pragma unroll
       for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) l += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[hb][r], kLog2e, -sh));
+        for (int r = 0; r < 16; ++r) l += split_exp(acc[hb][r], base);
       l += __shfl_xor(l, 32, 64);
       if (row_ok) {
         char* sp = reinterpret_cast<char*>(a.s) + E * (score_offset(a, pair, rt, n0 / 16) + 8 * lane);
@@ -211,11 +216,11 @@ __global__ __launch_bounds__(256) void split_score_kernel(SplitArgs a) {
       float mm = p[0][tid][0];
 #pragma unroll
       for (int j = 1; j < 4; ++j) mm = fmaxf(mm, p[j][tid][0]);
-      const float sh = (mm == -INFINITY ? 0.f : mm) * kLog2e;
+      const float base = mm == -INFINITY ? 0.f : mm;
       float ll = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        ll = __builtin_fmaf(p[j][tid][1], __builtin_amdgcn_exp2f(__builtin_fmaf(p[j][tid][0], kLog2e, -sh)), ll);
+        ll = __builtin_fmaf(p[j][tid][1], split_exp(p[j][tid][0], base), ll);
       float* st = a.stats + 2 * (((int64_t)pair * a.key_tiles + kt) * 32 * a.row_tiles + 32 * rt + tid);
       st[0] = mm;
       st[1] = ll;
@@ -239,7 +244,7 @@ __global__ __launch_bounds__(256) void split_value_kernel(SplitArgs a) {
   constexpr int SMEM = 4 * OB * 4096 > 8 * V_BYTES ? 4 * OB * 4096 : 8 * V_BYTES;
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
   __shared__ float sm[SG][ROWS], sl[SG][ROWS];
-  __shared__ float shl2e_[ROWS], inv_[ROWS];
+  __shared__ float base_[ROWS], inv_[ROWS];
   const int rgroups = (a.row_tiles + RT - 1) / RT;
   int x = blockIdx.x;
   const int rg = x % rgroups;
@@ -297,10 +302,10 @@ __global__ __launch_bounds__(256) void split_value_kernel(SplitArgs a) {
     lds_barrier();
 #pragma unroll
     for (int j = 0; j < SG; ++j) m = fmaxf(m, sm[j][r]);
-    const float sh = (m == -INFINITY ? 0.f : m) * kLog2e;
+    const float base = m == -INFINITY ? 0.f : m;
     float l = 0.f;
     auto add = [&](const f32x2_t& z) {
-      l = __builtin_fmaf(z[1], __builtin_amdgcn_exp2f(__builtin_fmaf(z[0], kLog2e, -sh)), l);
+      l = __builtin_fmaf(z[1], split_exp(z[0], base), l);
     };
 #pragma unroll
     for (int u = 0; u < SREG; ++u) add(y[u]);
@@ -312,15 +317,15 @@ __global__ __launch_bounds__(256) void split_value_kernel(SplitArgs a) {
 #pragma unroll
       for (int j = 1; j < SG; ++j) lt += sl[j][r];
       const bool dead = m == -INFINITY || lt == 0.f;
-      shl2e_[r] = sh;
+      base_[r] = base;
       inv_[r] = dead ? 0.f : 1.0f / lt;
     }
     lds_barrier();
   }
-  float shl2e[RT], inv[RT];
+  float base[RT], inv[RT];
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
-    shl2e[t] = shl2e_[32 * t + l32];
+    base[t] = base_[32 * t + l32];
     inv[t] = inv_[32 * t + l32];
   }
 
@@ -349,8 +354,7 @@ __global__ __launch_bounds__(256) void split_value_kernel(SplitArgs a) {
       float p[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(Num<T>::from_bits((sr[slot][t][e >> 1] >> (16 * (e & 1))) & 0xffffu),
-                                                     kLog2e, -shl2e[t])) * inv[t];
+        p[e] = split_exp(Num<T>::from_bits((sr[slot][t][e >> 1] >> (16 * (e & 1))) & 0xffffu), base[t]) * inv[t];
       pa[t] = u32x4_t{split_pack2<T>(p[0], p[1]), split_pack2<T>(p[2], p[3]), split_pack2<T>(p[4], p[5]),
                       split_pack2<T>(p[6], p[7])};
     }

@@ -122,6 +122,22 @@ def test_split_sdpa_is_batch_invariant(dtype, heads):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES16)
+def test_split_sdpa_masks_of_the_lowest_value(dtype):
+    """Padding written as the type's lowest value instead of -inf: whole wavefronts and workgroups of
+    keys in front, at the back, and all keys (which averages V)."""
+    q = randn(3, 8, 4, 64, seed=9250, dtype=dtype)
+    k, v = (randn(3, 2, 1100, 64, seed=9251 + i, dtype=dtype) for i in range(2))
+    mask = torch.zeros(3, 1, 4, 1100, dtype=dtype)
+    low = torch.finfo(dtype).min
+    mask[0, :, :, :700] = low
+    mask[1, :, :, 300:] = low
+    mask[2, :, 1] = low
+    out = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=mask.cuda(), enable_gqa=True)
+    check_sdpa(out, q, k, v, attn_mask=mask, what="lowest value", enable_gqa=True)
+
+
+@pytest.mark.gpu
 def test_split_sdpa_ignores_what_lies_past_the_keys():
     """Key and value rows past the end (NaN here) reach no output."""
     kc, vc = (torch.full((1, 2, 700, 64), math.nan, dtype=torch.bfloat16, device="cuda") for _ in "kv")
