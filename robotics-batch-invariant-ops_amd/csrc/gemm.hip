@@ -386,6 +386,65 @@ static int pick_cfg_f32(const BmmArgs& a) {
   return best;
 }
 
+// Grouped rows with a 16-bit N-major B on the direct path, more than kStreamMean rows per group on
+// average (the MoE expert GEMMs of a prefill): entries 0, 2, 11 and 22 by microseconds, rounds x (K
+// steps x per step + fixed), the tail launch of grouped_tail_rows included.  The 16-bit rates below
+// count rows only: a launch of few tiles took an entry of large tiles although every
+// entry's step has a floor (entry 2 1.0 us alone on its compute unit, 1.5 us in pairs; entry 0 1.85 and
+// 2.15; the streaming entry's deep ring 0.6).  Fitted on MI355X, bf16, K = 2048 with SwiGLU to N = 768 and
+// K = 768 to N = 2048, 8 experts at 32-384 rows each and 64 at 64-512, every entry forced (us, gate/up
+// and down): 8 experts of 64 rows entry 2 32.3 + 13.4, entry 22 21.3 + 9.8; of 128 36.4 + 14.2 / 21.9 +
+// 17.1; of 256, tails included, 56.6 + 23.5 / 39.8 + 25.4 (entry 11's down 17.7 without tails); 64
+// experts of 192 rows entry 2 148 + 83, entry 0 144 + 72, entry 22 213 + 118.
+constexpr int64_t kStreamMean = 56;
+struct GroupedCost {
+  int cfg, slots, bm, cols;       // slots: tiles of a round per compute unit; cols: B columns of a tile
+  double alone, loaded, fixed_alone, fixed;  // per K step with up to one tile per unit, and beyond
+};
+static const GroupedCost kGroupedCost[] = {
+    {0, 1, 256, 256, 1.85, 2.15, 3.0, 6.0},
+    {2, 2, 128, 128, 1.0, 1.5, 2.0, 4.0},
+    {11, 1, 128, 256, 1.25, 1.65, 2.0, 4.0},
+    {kStreamCfg + 2, 1, 64, 128, 0.63, 0.63, 1.2, 1.2},
+};
+static double grouped_us(const GroupedCost& g, double m_tiles, const BmmArgs& a, bool swiglu) {
+  const int64_t cus = device_cus();
+  const int64_t tiles = std::max<int64_t>(1, (int64_t)(m_tiles * (double)cdiv(a.N, swiglu ? g.cols / 2 : g.cols)));
+  const double steps = (double)(a.K / 64);
+  if (tiles <= cus) return steps * g.alone + g.fixed_alone;
+  return (double)cdiv(tiles, cus * g.slots) * (steps * g.loaded + g.fixed);
+}
+// Mean m-tiles of a group whose rows lie around the mean (20 % to either side).
+static double grouped_m_tiles(int64_t mean, int64_t bm) {
+  int64_t n = 0;
+  for (int p = 8; p <= 12; ++p) n += cdiv(std::max<int64_t>(1, mean * p / 10), bm);
+  return (double)n / 5.0;
+}
+// The cheaper of the launch with partial last m-tiles and the one that leaves last m-tiles of up to 63
+// rows to a tail launch (half of the groups taken to have one); `tails` says which.
+static double grouped_cost(const GroupedCost& g, const BmmArgs& a, bool swiglu, bool& tails) {
+  const int64_t groups = std::max<int64_t>(1, std::min(a.grp_groups, a.grp_rows)), mean = a.grp_rows / groups;
+  const double whole = grouped_us(g, (double)groups * grouped_m_tiles(mean, g.bm), a, swiglu);
+  tails = false;
+  if (g.bm < 128 || mean < 2 * g.bm) return whole;
+  const GroupedCost& stream = kGroupedCost[3];
+  const double split = grouped_us(g, (double)(groups * ((mean + g.bm - 65) / g.bm)), a, swiglu) +
+                       grouped_us(stream, (double)groups / 2, a, swiglu);
+  tails = split < whole;
+  return tails ? split : whole;
+}
+static int pick_cfg_grouped16(const BmmArgs& a, bool swiglu) {
+  int best = 2;
+  double best_us = 1e300;
+  for (const GroupedCost& g : kGroupedCost) {
+    if (swiglu && g.cfg == 11) continue;  // not built
+    bool tails;
+    const double us = grouped_cost(g, a, swiglu, tails);
+    if (us < best_us) { best_us = us; best = g.cfg; }
+  }
+  return best;
+}
+
 static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skinny_ok, bool nmajor16) {
   const bool swiglu = epi == kEpiSwiglu;
   const bool grouped = a.grp != nullptr;
@@ -464,7 +523,7 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skin
                     (dtype != BIOPS_F32 && row_blocks64 >= 2 && row_blocks64 <= 8 && a.K >= 1024 &&
                      row_blocks64 * cdiv(a.N, 64) <= cus)))
     best = kSkinnyCfg;
-  // Grouped rows of at most 56 rows per group on average with a 16-bit N-major B (the MoE
+  // Grouped rows of at most kStreamMean rows per group on average with a 16-bit N-major B (the MoE
   // expert GEMMs of calls up to about 7E/k tokens): the weight-streaming entries.  MI355X, C5
   // shapes (E = 64, D = 2048, I = 768, top-8), per sparse MoE call against the best table entry:
   // 1 token 47.1 us (16 rows) against 62.8 (entry 7); 2 tokens 56.3 against 74.5 (entry 2);
@@ -472,8 +531,10 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skin
   // tokens (32 rows per group) 160.1 (64 rows) against 170.8.  With the 128-column plain
   // blocks of 64-row m-tiles (same box): 384 tokens 167.3-173.0 against 173.8 (entry 2), 448
   // tokens 170.5 against 176.3; at 512 tokens entry 2 wins, 176.7 against 184.7.
-  if (stream_ok && mean <= 56)
+  if (stream_ok && mean <= kStreamMean)
     best = mean <= 2 ? kStreamCfg : mean <= 16 ? kStreamCfg + 1 : kStreamCfg + 2;
+  else if (stream_ok)
+    best = pick_cfg_grouped16(a, swiglu);
   return best;
 }
 
@@ -751,7 +812,8 @@ int grouped_tile_rows(int dtype, BmmArgs a, int epi, bool b_kmajor) {
   return cfg >= 0 && cfg < kNumCfg ? kCfgBM[cfg] : 0;
 }
 
-// Tails pay off only when the groups span two m-tiles or more on average: each tail streams its
+// Tails pay off only when the groups span two m-tiles or more on average and the partial m-tiles would
+// cost a round (grouped_cost): each tail streams its
 // group's whole B once more.  MI355X, C5 shapes (E = 64, D = 2048, I = 768, top-8), per sparse
 // MoE call, same box, with tails against without: 4096 tokens (512 rows per expert, 256-row
 // m-tiles) 471.3 against 496.3 us, 2048 tokens 323.1 against 319.7; without this condition
@@ -763,6 +825,11 @@ int grouped_tail_rows(int dtype, BmmArgs a, int epi, bool b_kmajor) {
   if (!direct || cfg < 0 || cfg >= kNumCfg || kCfgBM[cfg] < 128) return 0;
   const int64_t groups = std::max<int64_t>(1, std::min(a.grp_groups, a.grp_rows));
   if (a.grp_rows / groups < 2 * kCfgBM[cfg]) return 0;
+  if (forced_cfg() < 0 && a.grp_rows / groups > kStreamMean)  // (a forced entry keeps its tails)
+    for (const GroupedCost& g : kGroupedCost) {
+      bool tails;
+      if (g.cfg == cfg && (grouped_cost(g, a, epi == kEpiSwiglu, tails), !tails)) return 0;
+    }
   return kStreamBM[kNumStream - 1];
 }
 

@@ -285,3 +285,24 @@ def test_plan_over_512_chunks(quiet_index_watch):
     assert torch.count_nonzero(sparse[12345]) == 0 and torch.count_nonzero(sparse[T - 1]) == 0
     with pytest.raises(RuntimeError, match="outside"):
         check_moe_indices()
+
+
+# Rows per expert on both sides of the streaming entry's range and of the tail rule (8 experts: the
+# streaming entry up to 256 rows, 128-row m-tiles with their partial last ones above; 33 experts: tails)
+@pytest.mark.parametrize("T,E", [(228, 8), (700, 8), (1030, 8), (1530, 8), (2111, 8), (1300, 33), (8500, 33)])
+def test_grouped_entry_choice_gives_identical_bits(T, E):
+    dtype, D, I, k = torch.bfloat16, 512, 256, 2
+    hidden = randn(T, D, seed=8300 + T, dtype=dtype).cuda()
+    gate_up = randn(E, D, 2 * I, seed=8310 + E, dtype=dtype, scale=0.1).cuda()
+    down = randn(E, I, D, seed=8311 + E, dtype=dtype, scale=0.1).cuda().transpose(1, 2)
+    gate, up = gate_up[..., :I].transpose(1, 2), gate_up[..., I:].transpose(1, 2)
+    sel = torch.randint(0, E, (T, k), generator=torch.Generator().manual_seed(8320)).cuda()
+    sel[: T // 5] = E - 1  # one expert with most rows, others with few
+    w = torch.rand(T, k, generator=torch.Generator().manual_seed(8330)).cuda()
+    out = _moe(hidden, w, sel, gate, up, down, sparse=True)
+    lib = nat.load()
+    try:
+        assert lib.biops_set_gemm_tile(2) == 0
+        assert_bitwise(out, _moe(hidden, w, sel, gate, up, down, sparse=True), f"T={T} E={E}")
+    finally:
+        lib.biops_set_gemm_tile(-1)
