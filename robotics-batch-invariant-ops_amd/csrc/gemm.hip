@@ -228,7 +228,9 @@ void bmm_kernel(BmmArgs args) {
 
 // Computing wavefront w < CW of a skinny block stores its part straight from the accumulators
 // with the rounding of the LDS-staged epilogue: round(acc (+ bias[n])).
-template <typename S, typename T>
+// RB: with a row bias (a kernel of its own: the test for one at run time cost the few-row launches
+// 0.2 us of 8; built from 32-row blocks on).
+template <typename S, typename T, bool RB>
 __device__ __forceinline__ void skinny_store(const BmmArgs& args, const TileOrigin& o, int rows, int cols,
                                              const typename S::Acc& acc) {
   const int w = threadIdx.x >> 6;
@@ -236,14 +238,14 @@ __device__ __forceinline__ void skinny_store(const BmmArgs& args, const TileOrig
   const int wr = w / S::CWC, wc = w % S::CWC;
   const int64_t n0 = o.n0 + S::WC * wc;
   T* Cp = reinterpret_cast<T*>(args.C) + o.b1 * args.sC1 + o.b2 * args.sC2 + (o.m0 + S::WR * wr) * args.ldc + n0;
-  const T* bias = (args.bias && !args.row_bias) ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
+  const T* bias = (!RB && args.bias) ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
   const int wrows = rows - S::WR * wr, wcols = cols - S::WC * wc;
-  const T* row_bias = args.row_bias ? reinterpret_cast<const T*>(args.bias) + o.b2 * args.M + o.m0 + S::WR * wr : nullptr;
+  const T* row_bias = RB ? reinterpret_cast<const T*>(args.bias) + o.b2 * args.M + o.m0 + S::WR * wr : nullptr;
   S::Math::store(acc, Cp, args.ldc, wrows < S::WR ? wrows : S::WR, wcols < S::WC ? wcols : S::WC, bias, row_bias);
 }
 
 // One 32 x BC (or 64 x BC) block per workgroup.
-template <typename T, int AR, int BC>
+template <typename T, int AR, int BC, bool RB>
 __global__ __launch_bounds__(512) void skinny_kernel(BmmArgs args) {
   using S = SkinnyTile<T, AR, BC>;
   static_assert(S::THREADS == 512, "launch bounds");
@@ -259,12 +261,12 @@ __global__ __launch_bounds__(512) void skinny_kernel(BmmArgs args) {
   const int rows = rows64 < BH ? (int)rows64 : BH;
   const int cols = cols64 < BC ? (int)cols64 : BC;
   const typename S::Acc acc = S::run(smem, A, args.lda, rows, B, args.ldb, cols, args.K / S::BK);
-  skinny_store<S, T>(args, o, rows, cols, acc);
+  skinny_store<S, T, RB>(args, o, rows, cols, acc);
 }
 
 // The same blocks on the loader-split schedule (SkinnyTile::run_deep): CW computing and DL
 // loader wavefronts, K a whole number of 8-step stages (checked by the launcher).
-template <typename T, int AR, int BC>
+template <typename T, int AR, int BC, bool RB>
 __global__ __launch_bounds__((SkinnyTile<T, AR, BC>::DTHREADS)) void skinny_deep_kernel(BmmArgs args) {
   using S = SkinnyTile<T, AR, BC>;
   static_assert(S::DEEP && AR <= 32, "loader-split blocks of 32 rows");
@@ -279,7 +281,7 @@ __global__ __launch_bounds__((SkinnyTile<T, AR, BC>::DTHREADS)) void skinny_deep
   const int rows = rows64 < 32 ? (int)rows64 : 32;
   const int cols = cols64 < BC ? (int)cols64 : BC;
   const typename S::Acc acc = S::run_deep(smem, A, args.lda, rows, B, args.ldb, cols, args.K / S::BK);
-  skinny_store<S, T>(args, o, rows, cols, acc);
+  skinny_store<S, T, RB>(args, o, rows, cols, acc);
 }
 
 template <typename T, int BM, int BN, int SB, bool BKM>
@@ -538,8 +540,8 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skin
   return best;
 }
 
-template <typename T, int AR, int BC>
-static int launch_skinny_block(const BmmArgs& a0, hipStream_t stream) {
+template <typename T, int AR, int BC, bool RB>
+static int launch_skinny_rb(const BmmArgs& a0, hipStream_t stream) {
   BmmArgs a = a0;
   a.tiles_m = cdiv(a.M, AR > 32 ? 64 : 32);
   a.tiles_n = cdiv(a.N, BC);
@@ -553,12 +555,19 @@ static int launch_skinny_block(const BmmArgs& a0, hipStream_t stream) {
   if constexpr (S::DEEP) {
     const int64_t kt = a.K / S::BK;
     if (kt % S::UD == 0) {
-      hipLaunchKernelGGL((skinny_deep_kernel<T, AR, BC>), dim3((unsigned)grid), dim3(S::DTHREADS), 0, stream, a);
+      hipLaunchKernelGGL((skinny_deep_kernel<T, AR, BC, RB>), dim3((unsigned)grid), dim3(S::DTHREADS), 0, stream, a);
       return check_launch("skinny_deep_kernel");
     }
   }
-  hipLaunchKernelGGL((skinny_kernel<T, AR, BC>), dim3((unsigned)grid), dim3(S::THREADS), 0, stream, a);
+  hipLaunchKernelGGL((skinny_kernel<T, AR, BC, RB>), dim3((unsigned)grid), dim3(S::THREADS), 0, stream, a);
   return check_launch("skinny_kernel");
+}
+
+template <typename T, int AR, int BC>
+static int launch_skinny_block(const BmmArgs& a, hipStream_t stream) {
+  if constexpr (AR >= 32)
+    if (a.row_bias) return launch_skinny_rb<T, AR, BC, true>(a, stream);
+  return launch_skinny_rb<T, AR, BC, false>(a, stream);
 }
 
 // Block width: the narrowest of 8 / 16 / 32 / 64 columns whose blocks still fit one round on the
@@ -800,7 +809,7 @@ static int prepare_bmm(int dtype, BmmArgs& a, int epi, bool b_kmajor, bool& dire
            !direct_disabled();
   // Grouped rows run on the table entries only (the skinny and large-tile kernels take a fixed
   // tile count from the host); those two read K-major B only.
-  const bool skinny_ok = direct && b_kmajor && epi != kEpiSwiglu && a.grp == nullptr;
+  const bool skinny_ok = direct && b_kmajor && epi != kEpiSwiglu && a.grp == nullptr && !(a.row_bias && a.M <= 16);
   return pick_cfg(dtype, a, epi, direct, skinny_ok, direct && !b_kmajor && elt == 2);
 }
 
