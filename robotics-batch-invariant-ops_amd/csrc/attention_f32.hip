@@ -81,7 +81,11 @@ __device__ __forceinline__ float f32_merge_o(float o, float oc, float c1, float 
   const float t = oc * c2;
   return first ? t : __builtin_fmaf(o, c1, t);
 }
-__device__ __forceinline__ float f32_inverse(float l) { return l == 0.f ? 0.f : 1.0f / l; }
+// O / l at the end of a row; 0 where no score compares (all of them -inf or NaN), as the softmax kernels give.
+__device__ __forceinline__ f32x4_t f32_final(f32x4_t o, float m, float l) {
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  return m == -INFINITY || l == 0.f ? zero : o * (1.0f / l);
+}
 
 // MASK: 0 none, 1 boolean (bytes, nonzero = keep), 2 additive.  DP, DVP: head and value size rounded up
 // to 32 elements; QP: chunk pairs (8 elements) of the head size that are multiplied (zeros beyond).
@@ -320,7 +324,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
     if (row_ok && (some || last)) {
       float c1 = 1.f, c2 = 0.f;
       if (some) f32_merge(mt, lt, m, lc, c1, c2);
-      const float inv = last ? f32_inverse(lt) : 1.f;
 #pragma unroll
       for (int e = 0; e < OF; ++e) {
         f32x4_t o[4];  // a column block's loads before their first use (columns past dv read column 0)
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[j][i] = f32_merge_o(o[j][i], oacc[e][4 * j + i], c1, c2, first);
           }
-          if (col < a.dv) *reinterpret_cast<f32x4_t*>(orow + col) = last ? o[j] * inv : o[j];  // dv is a multiple of 4
+          if (col < a.dv) *reinterpret_cast<f32x4_t*>(orow + col) = last ? f32_final(o[j], mt, lt) : o[j];  // dv is a multiple of 4
         }
         __builtin_amdgcn_sched_barrier(0);  // one column block's registers at a time
       }
@@ -393,7 +396,7 @@ __global__ __launch_bounds__(256) void f32_combine_kernel(F32AttnArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = f32_merge_o(o[e], oc[e], c1, c2, first);
   }
-  *reinterpret_cast<f32x4_t*>(a.out + r * a.dv + col) = o * f32_inverse(l);
+  *reinterpret_cast<f32x4_t*>(a.out + r * a.dv + col) = f32_final(o, m, l);
 }
 
 template <int DP, int QP, int DVP, bool SPLIT>
