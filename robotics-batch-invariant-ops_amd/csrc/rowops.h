@@ -102,14 +102,32 @@ __device__ __forceinline__ void store_row_chunk(T* row, int64_t cols, int64_t c0
     if (c0 + e < cols) Num<T>::store(row + c0 + e, v[e]);
 }
 
-// exp(x - shift) for the softmax family: the accurate libm expf when the result is stored as
-// fp32; when it is rounded to 16 bits anyway, the hardware exp2 of fma(x, log2 e, -shift log2 e)
-// (`shl2e` = shift * log2 e, computed once per row).
+// exp(x - m) for the softmax family, m the row's maximum (or 0 for a row of -inf): the accurate libm
+// expf when the result is stored as fp32; when it is rounded to 16 bits anyway, the hardware exp2
+// of fma(x, log2 e, -m log2 e).  The rounding of m log2 e is common to the row and cancels in the
+// division by the row sum while it is small; a row whose maximum is huge (masked with the type's
+// lowest value, where the product overflows) takes the difference first instead.
 constexpr float kLog2e = 1.4426950408889634f;
-template <typename Tout>
-__device__ __forceinline__ float soft_exp(float x, float shift, float shl2e) {
-  if constexpr (sizeof(Tout) == 4) return expf(x - shift);
-  else return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, -shl2e));
+struct SoftShift {
+  float m, ml2e;
+  bool wide;  // |m log2 e| >= 2^16 (its rounding is 2^-8 and more), the same in the whole wavefront
+};
+__device__ __forceinline__ SoftShift soft_shift(float m) {
+  const float ml2e = m * kLog2e;
+  return SoftShift{m, ml2e, (bool)__any(fabsf(ml2e) >= 65536.f)};
+}
+template <typename Tout, int N>
+__device__ __forceinline__ void soft_exp(float (&v)[N], const SoftShift& s) {
+  if constexpr (sizeof(Tout) == 4) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = expf(v[e] - s.m);
+  } else if (__builtin_expect(s.wide, 0)) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f((v[e] - s.m) * kLog2e);
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[e], kLog2e, -s.ml2e));
+  }
 }
 
 // ------------------------------------------------------------------ softmax rows ----
@@ -179,8 +197,7 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
   }
   mx = wave_max(mx);
   const bool all_neg_inf = (mx == -INFINITY);
-  const float shift = all_neg_inf ? 0.f : mx;
-  const float shl2e = shift * kLog2e;
+  const SoftShift shift = soft_shift(all_neg_inf ? 0.f : mx);
 
   float sum = 0.f;
   if (fits) {
@@ -188,9 +205,10 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
     for (int j = 0; j < kRowRegChunks; ++j) {
       const int64_t ci = lane + 64 * j;
       if (ci < nchunks) {
+        soft_exp<T>(cache[j], shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          cache[j][e] = all_neg_inf ? 0.f : soft_exp<T>(cache[j][e], shift, shl2e);
+          if (all_neg_inf) cache[j][e] = 0.f;
           if (ci * VEC + e < cols) sum += cache[j][e];
         }
       }
@@ -200,11 +218,10 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
       float v[VEC];
       load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
       transform_chunk<T>(ar, ci * VEC, cols, v);
+      soft_exp<T>(v, shift);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        const float ex = all_neg_inf ? 0.f : soft_exp<T>(v[e], shift, shl2e);
-        if (ci * VEC + e < cols) sum += ex;
-      }
+      for (int e = 0; e < VEC; ++e)
+        if (ci * VEC + e < cols) sum += all_neg_inf ? 0.f : v[e];
     }
   }
   sum = wave_sum(sum);
@@ -227,11 +244,10 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
       float v[VEC];
       load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
       transform_chunk<T>(ar, ci * VEC, cols, v);
-      float o[VEC];
+      soft_exp<T>(v, shift);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e)
-        o[e] = zero ? 0.f : (all_neg_inf ? 0.f : soft_exp<T>(v[e], shift, shl2e)) * inv;
-      store_row_chunk<T, VEC>(row, cols, ci * VEC, o);
+      for (int e = 0; e < VEC; ++e) v[e] = zero || all_neg_inf ? 0.f : v[e] * inv;
+      store_row_chunk<T, VEC>(row, cols, ci * VEC, v);
     }
   }
 }
@@ -281,18 +297,20 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     neg_inf[r] = (mx[r] == -INFINITY);
-    const float shift = (MODE == kLogSoftmax || !neg_inf[r]) ? mx[r] : 0.f;
-    const float shl2e = shift * kLog2e;
+    const SoftShift shift = soft_shift((MODE == kLogSoftmax || !neg_inf[r]) ? mx[r] : 0.f);
     sum[r] = 0.f;
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const int64_t ci = lane + 64 * j;
       if (ci < nchunks) {
+        float ex[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) ex[e] = cache[r][j][e];
+        soft_exp<Tout>(ex, shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          const float ex = (MODE != kLogSoftmax && neg_inf[r]) ? 0.f : soft_exp<Tout>(cache[r][j][e], shift, shl2e);
-          if (MODE != kLogSoftmax) cache[r][j][e] = ex;
-          if (ci * VEC + e < cols) sum[r] += ex;
+          if (MODE != kLogSoftmax) cache[r][j][e] = ex[e] = neg_inf[r] ? 0.f : ex[e];
+          if (ci * VEC + e < cols) sum[r] += ex[e];
         }
       }
     }

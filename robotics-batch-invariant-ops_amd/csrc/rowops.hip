@@ -92,10 +92,12 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
     }
   };
   // exp of a column past the row end is 0 (NaN only where the whole row gives NaN)
-  auto exps = [&](float (&v)[VEC], bool neg_inf, float shift, float shl2e) {
+  auto exps = [&](float (&v)[VEC], bool neg_inf, const SoftShift& shift) {
+    soft_exp<Tout>(v, shift);
+    if (MODE != kLogSoftmax && neg_inf) {
 #pragma unroll
-    for (int e = 0; e < VEC; ++e)
-      v[e] = (MODE != kLogSoftmax && neg_inf) ? 0.f : soft_exp<Tout>(v[e], shift, shl2e);
+      for (int e = 0; e < VEC; ++e) v[e] = 0.f;
+    }
   };
 
   float mx = -INFINITY;
@@ -112,8 +114,7 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
   mx = block_max<NW>(mx, part[0]);
   keep_raw();
   const bool neg_inf = (mx == -INFINITY);
-  const float shift = (MODE == kLogSoftmax || !neg_inf) ? mx : 0.f;
-  const float shl2e = shift * kLog2e;
+  const SoftShift shift = soft_shift((MODE == kLogSoftmax || !neg_inf) ? mx : 0.f);
 
   // fp32 softmax of a resident row keeps the exponentials in the row's registers
   constexpr bool kKeepExp = !LOOP && sizeof(Tin) == 4 && MODE == kSoftmax;
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
     for (int j = 0; j < NC; ++j) {
       float v[VEC];
       unpack_chunk<Tin>(raw[j], v);
-      exps(v, neg_inf, shift, shl2e);
+      exps(v, neg_inf, shift);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) sum += v[e];
       if constexpr (kKeepExp) {
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) v[e] = v[e] - mx - lse;
       } else {
-        if constexpr (!kKeepExp) exps(v, neg_inf, shift, shl2e);
+        if constexpr (!kKeepExp) exps(v, neg_inf, shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) v[e] = zero ? 0.f : v[e] * inv;
       }

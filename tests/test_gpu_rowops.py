@@ -206,3 +206,24 @@ def test_long_rows_mean_and_norm(dtype, chunks, extra):
         assert_close_scaled(out, ref, rel=REL[dtype], abs_scale=1e-7, what=f"{cols}")
         assert_bitwise(fn(gx[1:2], -1), out[1:2], "row 1 alone")
         assert_bitwise(fn(shifted[1:].view(3, cols), -1), out, "misaligned rows")
+
+
+@pytest.mark.parametrize("dtype_in,dtype_out", ((torch.bfloat16, None), (torch.float32, torch.bfloat16),
+                                                (torch.float32, torch.float16), (torch.float32, None)))
+@pytest.mark.parametrize("cols", (8, 300, 2048, 4103, 40000, 200003))
+def test_softmax_rows_of_the_lowest_value(dtype_in, dtype_out, cols):
+    """A row whose maximum is the type's lowest value (whose multiple by log2 e overflows) is as uniform as
+    any other constant row; other keys beside such values take the whole weight."""
+    low = torch.finfo(dtype_in).min
+    x = torch.full((4, cols), low, dtype=dtype_in, device="cuda")
+    x[1] = -1e9
+    x[2, 1:] = 0.0
+    x[3, cols // 2] = -math.inf
+    p = softmax(x, -1, dtype=dtype_out)
+    ref = torch.softmax(x.double(), -1)
+    assert torch.equal(p, ref.to(p.dtype)) or torch.allclose(p.double(), ref, rtol=2.0**-7, atol=2.0**-24)
+    if dtype_out is None:
+        logp = log_softmax(x, -1)
+        ref = torch.log_softmax(x.double(), -1)
+        # x - max - log(sum): the two roundings of a bf16 output's fp32 value and the output's own
+        assert torch.allclose(logp.double(), ref, rtol=2.0**-8 if dtype_in == torch.bfloat16 else 2.0**-20)
