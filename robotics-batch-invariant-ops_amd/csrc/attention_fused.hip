@@ -29,8 +29,8 @@
 #include <cstdlib>
 #include <vector>
 
+#include "attention16.h"
 #include "gemm.h"
-#include "rowops.h"
 
 namespace biops {
 
@@ -448,13 +448,12 @@ void fused_attn_kernel(FusedArgs a) {
 #pragma unroll
     for (int r = 1; r < 16; ++r) bm = fmaxf(bm, sc[r]);
     bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
-    // m = -inf until a visible key appears: the shift stays 0 and every term is exp(-inf) = 0
     const float mn = fmaxf(m, bm);
-    const float sh = (mn == -INFINITY ? 0.f : mn) * kexp;
-    const float corr = __builtin_amdgcn_exp2f(__builtin_fmaf(m, kexp, -sh));
+    const ExpBase base = attn_exp_base<T, MASK == 2>(mn, kexp);
+    const float corr = attn_rescale(m, base);
     float part = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) part += __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], kexp, -sh));
+    for (int r = 0; r < 16; ++r) part += attn_exp(sc[r], base);
     l = __builtin_fmaf(l, corr, part);
     m = mn;
   };
@@ -497,7 +496,7 @@ void fused_attn_kernel(FusedArgs a) {
   const float lt = l + __shfl_xor(l, 32, 64);
   const bool dead = (m == -INFINITY) || (lt == 0.f);
   const float inv = dead ? 0.f : 1.0f / lt;
-  const float shl2e = (m == -INFINITY ? 0.f : m) * kexp;
+  const ExpBase base = attn_exp_base<T, MASK == 2>(m, kexp);
 
   // ---------------------------------------------------------------- pass 2: P V ----
   f32x16_t oacc[F::OF];
@@ -523,8 +522,7 @@ void fused_attn_kernel(FusedArgs a) {
       // 16-key chunk c = 2 hb + c2: this lane's keys 16c + 4hf + (0..3) and + 8
       float p[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * c2 + e], kexp, -shl2e)) * inv;
+      for (int e = 0; e < 8; ++e) p[e] = attn_exp(sc[8 * c2 + e], base) * inv;
       const u32x4_t pa = {pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3]), pack2<T>(p[4], p[5]),
                           pack2<T>(p[6], p[7])};
       const int row = 16 * (2 * hb + c2) + vrow;
@@ -626,7 +624,7 @@ static int launch_fused(int dtype, const FusedArgs& a, hipStream_t s) {
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // scale = 2^k with -8 <= k <= 0 (the fused kernels' exact power-of-two path); the environment
 // variable BIOPS_ATTN_GENERIC_SCALE=1 turns the path off (tests compare the two).
-static int pow2_scale(float scale) {
+int pow2_scale(float scale) {
   int e = 0;
   if (!(scale > 0.f) || std::frexp(scale, &e) != 0.5f || e - 1 < -8 || e - 1 > 0) return 0;
   const char* env = std::getenv("BIOPS_ATTN_GENERIC_SCALE");

@@ -141,6 +141,26 @@ def test_fused_sdpa_masks(mask_kind, dtype, lk, materialized):
     assert_first_sample_equal(alone, out)
 
 
+@pytest.mark.parametrize("dtype,huge", ((torch.bfloat16, torch.finfo(torch.bfloat16).min), (torch.bfloat16, -1e9),
+                                        (torch.bfloat16, -7e4), (torch.float16, torch.finfo(torch.float16).min)))
+def test_sdpa_masks_of_huge_values(dtype, huge, materialized):
+    """Padding written as the type's lowest value or as a large negative number instead of -inf: the
+    first keys of a row, the last ones, and all of them (which averages V)."""
+    B, Hq, Lq, Lk, D = 3, 4, 150, 2600, 64
+    q = randn(B, Hq, Lq, D, seed=4600, dtype=dtype)
+    k, v = (randn(B, 2, Lk, D, seed=4601 + i, dtype=dtype) for i in range(2))
+    mask = torch.zeros(B, 1, Lq, Lk, dtype=dtype)
+    mask[0, :, :, :700] = huge
+    mask[1, :, :, 300:] = huge
+    mask[2, :, ::3] = huge
+    mask[2, :, 1::3, :32] = huge
+    kw = dict(enable_gqa=True)
+    dev = (q.cuda(), k.cuda(), v.cuda())
+    fused = sdpa(*dev, attn_mask=mask.cuda(), **kw)
+    check_sdpa(fused, q, k, v, attn_mask=mask, what="fused", **kw)
+    check_sdpa(materialized(sdpa, *dev, attn_mask=mask.cuda(), **kw), q, k, v, attn_mask=mask, what="materialised", **kw)
+
+
 def test_fused_sdpa_per_head_mask_and_gqa_equals_repeat():
     dtype = torch.bfloat16
     q = randn(1, 8, 96, 64, seed=8250, dtype=dtype).cuda()
