@@ -235,10 +235,9 @@ int biops_sdpa_fused(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t 
                      const void* mask, int mask_dtype, int64_t mB, int64_t mH, int64_t mI, int64_t mJ,
                      int causal, float scale, void* out, void* stream);
 
-/* Same operator as biops_sdpa_fused without causal masking, for few query rows (lq <= 16) against
- * more than 512 keys: the keys are split over workgroups, with 16-bit scores, row statistics and
- * fp32 partial outputs in a workspace.  Same roundings; S is bitwise the materialised S, the row
- * sum and the P V sum run in an order that depends on lk only.
+/* Same operator and bits as biops_sdpa_fused without causal masking, for few query rows (lq <= 16)
+ * against more than 512 keys: keys (scores), then rows and value columns (row statistics and P V) are
+ * spread over workgroups, with the 16-bit scores and their maxima per 32 keys in a workspace.
  * biops_sdpa_split_workspace_size: workspace bytes, or -1 when biops_sdpa_split does not take the
  * call (dtype, head sizes, causal, query rows, key count).  The workspace is 256-byte aligned, out
  * a contiguous [batch, hq, lq, dv]; layout conditions as biops_sdpa_fused.

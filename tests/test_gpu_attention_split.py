@@ -103,6 +103,60 @@ def test_split_sdpa_matches_oracle_and_materialized(dtype, mask_kind, shape, mon
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DTYPES16)
+@pytest.mark.parametrize("mask_kind", ("none", "boolean", "additive", "lowest"))
+@pytest.mark.parametrize("shape", SHAPES + ((1, 2, 1, 3, 9000, 64, 128), (40, 14, 2, 5, 1029, 128, 136)))
+def test_query_rows_in_chunks_give_the_bits_of_one_call(dtype, mask_kind, shape):
+    """A row's bits are the same in a call of up to 16 query rows (split) and in a longer one (fused)."""
+    B, Hq, Hkv, Lq, Lk, D, Dv = shape
+    if mask_kind != "none":
+        Lk = -(-Lk // 4) * 4
+    seed = 9450 + Lk
+    q = randn(B, Hq, Lq + 30, D, seed=seed, dtype=dtype).cuda()
+    k = (randn(B, Hkv, Lk, D, seed=seed + 1, dtype=dtype) * torch.linspace(0.2, 3, Lk).view(-1, 1).to(dtype)).cuda()
+    v = randn(B, Hkv, Lk, Dv, seed=seed + 2, dtype=dtype).cuda()
+    mask = None
+    if mask_kind != "none":
+        g = torch.Generator().manual_seed(seed + 3)
+        mask = torch.rand(B, 1, Lq + 30, Lk, generator=g) > 0.2
+        mask[:, :, Lq // 2] = False
+        mask[0, :, :, : Lk // 2] = False
+        if mask_kind != "boolean":
+            keep = mask
+            mask = (torch.rand(B, 1, Lq + 30, Lk, generator=g) * -10).to(dtype)
+            mask[~keep] = -math.inf if mask_kind == "additive" else torch.finfo(dtype).min
+        mask = mask.cuda()
+    assert size(B, Hq, Hkv, Lq, Lk, D, Dv) > 0 and size(B, Hq, Hkv, Lq + 30, Lk, D, Dv) < 0
+    for scale in (None, 0.3):
+        whole = sdpa(q, k, v, attn_mask=mask, scale=scale, enable_gqa=Hq != Hkv)
+        for first in (0, 13):
+            rows = slice(first, first + Lq)
+            part = sdpa(q[:, :, rows], k, v, attn_mask=None if mask is None else mask[:, :, rows], scale=scale,
+                        enable_gqa=Hq != Hkv)
+            assert_bitwise(part, whole[:, :, rows], f"rows from {first}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES16)
+def test_infinities_and_nan_in_chunks_of_query_rows(dtype):
+    """NaN and infinite queries, keys and values reach the same outputs at any number of query rows."""
+    q = randn(4, 4, 40, 64, seed=9480, dtype=dtype).cuda()
+    k, v = (randn(4, 2, 1100, 64, seed=9481 + i, dtype=dtype).cuda() for i in range(2))
+    q[0, 1, 3] = math.nan
+    k[1, 0, 70:200] = math.nan
+    k[2, 1, 500, 0] = math.inf
+    v[3, 0, 5] = math.nan
+    v[3, 1, 1099] = math.inf
+    mask = torch.ones(4, 1, 1, 1100, dtype=torch.bool, device="cuda")
+    mask[3, ..., 1000:] = False
+    for m in (None, mask):
+        whole = sdpa(q, k, v, attn_mask=m, enable_gqa=True)
+        part = sdpa(q[:, :, :7], k, v, attn_mask=m, enable_gqa=True)
+        assert torch.equal(part.isnan(), whole[:, :, :7].isnan())
+        assert_bitwise(part.nan_to_num(1.0), whole[:, :, :7].nan_to_num(1.0), "finite outputs")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES16)
 @pytest.mark.parametrize("heads", ((16, 4, 1), (64, 8, 16), (8, 8, 5)))
 def test_split_sdpa_is_batch_invariant(dtype, heads):
     """Samples alone and in a batch large enough for several row tiles per workgroup; the batch is
