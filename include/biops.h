@@ -239,9 +239,11 @@ int biops_sdpa_fused(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t 
  * against more than 512 keys: keys (scores), then rows and value columns (row statistics and P V) are
  * spread over workgroups, with the 16-bit scores and their maxima per 32 keys in a workspace.
  * biops_sdpa_split_workspace_size: workspace bytes, or -1 when biops_sdpa_split does not take the
- * call (dtype, head sizes, causal, query rows, key count).  The workspace is 256-byte aligned, out
- * a contiguous [batch, hq, lq, dv]; layout conditions as biops_sdpa_fused.
+ * call (dtype, head sizes, causal, query rows, key count, a workspace over 2 GiB): biops_sdpa_fused
+ * takes it.  The workspace is 256-byte aligned, out a contiguous [batch, hq, lq, dv]; layout
+ * conditions as biops_sdpa_fused.  biops_sdpa_split_max_query: the query rows it takes at most.
  * Replaces scaled_dot_product_attention_batch_invariant (batch_invariant_ops.py:1148-1213). */
+int biops_sdpa_split_max_query(void);
 int64_t biops_sdpa_split_workspace_size(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t lq,
                                         int64_t lk, int64_t d, int64_t dv, int causal);
 int biops_sdpa_split(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk,

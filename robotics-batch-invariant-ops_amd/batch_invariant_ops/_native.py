@@ -71,6 +71,7 @@ _SIGNATURES = {
         + [_p, _l, _l, _l] * 3
         + [_p, _i, _l, _l, _l, _l, _i, _f, _p, _p],
     ),
+    "biops_sdpa_split_max_query": (_i, []),
     "biops_sdpa_split_workspace_size": (_l, [_i, _l, _l, _l, _l, _l, _l, _l, _i]),
     "biops_sdpa_split": (
         _i,

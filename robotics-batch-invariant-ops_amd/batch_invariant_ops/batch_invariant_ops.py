@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import math
 import threading
 from collections import namedtuple
@@ -625,8 +626,18 @@ def _sdpa_glue(q4, k4, v4, group, mask4, scale, out_dtype):
     return bmm_persistent(probabilities.reshape(B * Hq, Lq, Lk), v4.reshape(B * Hq, Lk, v4.shape[-1]))
 
 
-# Query rows up to which biops_sdpa_split_workspace_size is asked (the library's own limit).
-_SPLIT_MAX_QUERY = 16
+@functools.lru_cache(maxsize=None)
+def _split_max_query():
+    """Query rows up to which ``biops_sdpa_split`` is worth asking."""
+    return nat.load().biops_sdpa_split_max_query()
+
+
+def _workspace_or_none(nbytes, device):
+    """A workspace for a path that the caller can do without; None when the memory is not there."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def scaled_dot_product_attention_batch_invariant(
@@ -710,11 +721,11 @@ def scaled_dot_product_attention_batch_invariant(
     fused = _fused_attention_ok(query.dtype, D, Dv, q4, k4, v4)
     if fused and mask4 is not None:
         fused = bool(nat.load().biops_attention_fused_mask_ok(mask4.data_ptr(), mask_code, Lk, *mask4.stride()))
-    if fused and Lq <= _SPLIT_MAX_QUERY:
+    if fused and Lq <= _split_max_query():
         ws_bytes = _fast_fn("biops_sdpa_split_workspace_size")(
             nat.dtype_code(query.dtype), B, Hq, Hkv, Lq, Lk, D, Dv, causal_code)
-        if ws_bytes >= 0:
-            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
+        workspace = _workspace_or_none(ws_bytes, query.device) if ws_bytes >= 0 else None
+        if workspace is not None:
             rc = _fast_fn("biops_sdpa_split")(
                 nat.dtype_code(query.dtype), B, Hq, Hkv, Lq, Lk, D, Dv,
                 q4.data_ptr(), q4.stride(0), q4.stride(1), q4.stride(2),

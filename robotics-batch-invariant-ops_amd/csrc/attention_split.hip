@@ -50,6 +50,9 @@ constexpr int kSplitKeys = 256;      // keys per workgroup of split_score_kernel
 //   host time, so calls up to 512 keys, which the host bounds either way, stay on the fused kernel.
 constexpr int kSplitMaxQuery = 16;   // query rows per head
 constexpr int kSplitMinKeys = 512;   // longer key ranges are split
+// The fused kernel needs no workspace, so this path must not make a call run out of memory that
+// fitted: larger calls stay there (512 pairs of up to 32 rows take 2 GiB at 60000 keys).
+constexpr int64_t kSplitMaxWorkspace = int64_t(2) << 30;
 
 struct SplitArgs {
   const void* q; const void* k; const void* v; void* out;
@@ -602,8 +605,10 @@ extern "C" int64_t biops_sdpa_split_workspace_size(int dtype, int64_t batch, int
   if (lk >= (int64_t(1) << 30) || z.rows >= (int64_t(1) << 25) ||
       batch * hkv >= lim / (2 * std::max<int64_t>(z.key_tiles, 4) * z.row_tiles))
     return -1;
-  return z.total;
+  return z.total <= kSplitMaxWorkspace ? z.total : -1;
 }
+
+extern "C" int biops_sdpa_split_max_query(void) { return kSplitMaxQuery; }
 
 extern "C" int biops_sdpa_split(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk, int64_t d,
                                 int64_t dv, const void* q, int64_t sqB, int64_t sqH, int64_t sqL, const void* k,

@@ -36,6 +36,30 @@ def test_which_calls_are_split():
         assert size(batch, 16, 4, 1, 4096, dtype=nat.F32) < 0
         assert size(batch, 16, 4, 1, 4096, D=264) < 0 and size(batch, 16, 4, 1, 4096, Dv=12) < 0
     assert size(1, 16, 3, 1, 4096) < 0 and size(0, 16, 4, 1, 4096) < 0
+    assert nat.load(require_gpu=False).biops_sdpa_split_max_query() == 16
+
+
+def test_large_workspaces_are_left_to_the_fused_kernel():
+    """Which path runs changes no bit, so the batch may enter here: 2 GiB at most."""
+    assert 0 < size(64, 64, 8, 1, 32768) <= 2 << 30
+    assert size(64, 64, 8, 16, 32768) < 0 and size(1, 8, 8, 1, 1 << 23) < 0
+    assert size(1 << 20, 64, 64, 16, 4096) < 0  # also past the launch limits
+
+
+@pytest.mark.gpu
+def test_without_memory_for_the_workspace(monkeypatch):
+    q = randn(2, 8, 3, 64, seed=9430, dtype=torch.bfloat16).cuda()
+    k, v = (randn(2, 2, 700, 64, seed=9431 + i, dtype=torch.bfloat16).cuda() for i in range(2))
+    out = sdpa(q, k, v, enable_gqa=True)
+    empty = torch.empty
+
+    def refuse(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no workspace")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", refuse)
+    assert_bitwise(sdpa(q, k, v, enable_gqa=True), out, "fused kernel instead")
 
 
 def test_argument_errors_come_before_any_launch():
