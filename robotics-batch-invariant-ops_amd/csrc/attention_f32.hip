@@ -59,10 +59,19 @@ struct F32AttnArgs {
   float* stats;
 };
 
-// exp(x - m).  The difference is taken before the factor log2 e: a row of which every key carries a
-// mask of the type's lowest value has a finite maximum whose multiple by log2 e is not (fma(x, log2 e,
-// -m log2 e) gave NaN there).
-__device__ __forceinline__ float f32_exp(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * kLog2e); }
+// exp(x - m), x <= m, to the accuracy of expf (whose place it takes: the fp32 softmax has expf).  With d =
+// x - m: e = round(d log2 e), 2^e * exp2(d log2 e - e), the difference from log2 e in two parts, so its
+// error stays near 2^-25 at any d (the exp2 of the rounded product alone is off by |d| 2^-24 and
+// flushes below 2^-126).  e is kept at -160 and above, where everything is 0: -inf gives 0, NaN
+// comes through the difference.  8 x 16 x 256 x 256, head size 72: 40.9 us with expf, 39.3 so,
+// 37.8 with the plain exp2.
+__device__ __forceinline__ float f32_exp(float x, float m) {
+  constexpr float kLow = 1.925963e-8f;  // log2 e - kLog2e
+  const float d = x - m;
+  const float e = fmaxf(__builtin_rintf(d * kLog2e), -160.f);
+  const float a = __builtin_fmaf(d, kLow, __builtin_fmaf(d, kLog2e, -e));
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(a), (int)e);
+}
 
 // False for a chunk without a visible key.  A chunk whose scores are all NaN has the maximum -inf too,
 // but a NaN sum.

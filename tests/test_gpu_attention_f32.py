@@ -159,3 +159,18 @@ def test_f32_sdpa_passes_nan_on(B, monkeypatch):
     assert out[:, 0].isfinite().all() and out[:, 3].isfinite().all()
     monkeypatch.setenv("BIOPS_ATTENTION_MATERIALIZE", "1")
     assert torch.equal(sdpa(q, k, v).isnan(), out.isnan())
+
+
+@pytest.mark.gpu
+def test_f32_sdpa_probabilities_to_the_last_bits():
+    """Two keys with scores 0 and -x: the output is exp(-x) / (1 + exp(-x)).  expf is within 1 ulp, the sum,
+    the reciprocal and the product round once more each: under 4 ulps, 2^-21 of the value (taking the
+    exponential of a rounded multiple of x was off by up to x 2^-24 more)."""
+    x = torch.linspace(0.0, 86.0, 1024)
+    q, k, v = (torch.zeros(1, 1, n, 4) for n in (1024, 2, 2))
+    q[0, 0, :, 0] = x
+    k[0, 0, 1, 0] = -1.0
+    v[0, 0, 1] = 1.0
+    out = sdpa(q.cuda(), k.cuda(), v.cuda(), scale=1.0)
+    ref = torch.sigmoid(-x.double())[:, None].expand(-1, 4)
+    assert torch.allclose(out[0, 0].cpu().double(), ref, rtol=2.0**-21, atol=0.0)
