@@ -599,15 +599,22 @@ def _fused_attention_ok(dtype, d, dv, *tensors, varlen=False):
     return True
 
 
-def _f32_attention_ok(B, Hq, Lq, Lk, D, Dv, *tensors):
-    """True when the one-pass float32 kernel takes this call (head sizes multiples of 4 up to 128,
-    16-byte aligned rows); ``BIOPS_ATTENTION_MATERIALIZE=1`` selects the materialised path."""
-    if not nat.load().biops_sdpa_f32_supported(B, Hq, Lq, Lk, D, Dv):
-        return False
-    if nat.env_flag("BIOPS_ATTENTION_MATERIALIZE", False):
-        return False
-    return not any(t.data_ptr() % 16 or t.stride(2) >= 1 << 25 or any(st % 4 for st in t.stride()[:-1])
-                   for t in tensors)
+def _f32_attention_ok(B, Hq, Lq, Lk, D, Dv):
+    """True when the one-pass float32 kernel takes this call (head sizes multiples of 4 up to 128);
+    ``BIOPS_ATTENTION_MATERIALIZE=1`` selects the materialised path.  The sizes alone decide: the two
+    paths sum in another order, and a view must give the bits of its copy."""
+    return bool(nat.load().biops_sdpa_f32_supported(B, Hq, Lq, Lk, D, Dv)) and not nat.env_flag(
+        "BIOPS_ATTENTION_MATERIALIZE", False)
+
+
+def _f32_rows(t):
+    """``t`` [B, H, L, D] with the 16-byte aligned rows that the one-pass float32 kernel reads, copied
+    where a view has others, and its strides (0 for dimensions of one element)."""
+    strides = [st if n > 1 else 0 for n, st in zip(t.shape[:-1], t.stride())]
+    if t.data_ptr() % 16 or strides[2] >= 1 << 25 or any(st % 4 for st in strides):
+        t = t.clone(memory_format=torch.contiguous_format)
+        strides = t.stride()[:-1]
+    return t, strides
 
 
 def _sdpa_glue(q4, k4, v4, group, mask4, scale, out_dtype):
@@ -749,14 +756,13 @@ def scaled_dot_product_attention_batch_invariant(
         )
         nat.check(rc, "biops_sdpa_fused")
         return out.reshape(*leading, Lq, Dv)
-    if query.dtype == torch.float32 and _f32_attention_ok(B, Hq, Lq, Lk, D, Dv, q4, k4, v4):
+    if query.dtype == torch.float32 and _f32_attention_ok(B, Hq, Lq, Lk, D, Dv):
         ws_bytes = nat.load().biops_sdpa_f32_workspace_size(B, Hq, Lq, Lk, D, Dv)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
+        (qr, sq), (kr, sk), (vr, sv) = _f32_rows(q4), _f32_rows(k4), _f32_rows(v4)
         rc = _fast_fn("biops_sdpa_f32")(
             B, Hq, Hkv, Lq, Lk, D, Dv,
-            q4.data_ptr(), q4.stride(0), q4.stride(1), q4.stride(2),
-            k4.data_ptr(), k4.stride(0), k4.stride(1), k4.stride(2),
-            v4.data_ptr(), v4.stride(0), v4.stride(1), v4.stride(2),
+            qr.data_ptr(), *sq, kr.data_ptr(), *sk, vr.data_ptr(), *sv,
             mask4.data_ptr() if mask4 is not None else None, mask_code,
             *(mask4.stride() if mask4 is not None else (0, 0, 0, 0)),
             causal_code, float(scale_value), out.data_ptr(),

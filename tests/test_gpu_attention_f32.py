@@ -174,3 +174,30 @@ def test_f32_sdpa_probabilities_to_the_last_bits():
     out = sdpa(q.cuda(), k.cuda(), v.cuda(), scale=1.0)
     ref = torch.sigmoid(-x.double())[:, None].expand(-1, 4)
     assert torch.allclose(out[0, 0].cpu().double(), ref, rtol=2.0**-21, atol=0.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ("base", "pitch", "keys", "wide"))
+def test_f32_sdpa_views_give_the_bits_of_their_copies(layout):
+    """Rows that are not 16-byte aligned (an offset base, an odd pitch, keys behind an odd offset) and
+    rows further apart than the kernel's 32-bit offsets take the same path as an aligned copy."""
+    B, H, L, D = 3, 2, 200, 64
+
+    def view(seed):
+        if layout == "base":
+            return randn(B * H * L * D + 1, seed=seed).cuda()[1:].view(B, H, L, D)
+        if layout == "pitch":
+            return randn(B, L, H, D + 1, seed=seed).cuda()[..., :D].transpose(1, 2)
+        if layout == "keys":
+            return randn(B, H, L * D + 3, seed=seed).cuda()[..., 3:].view(B, H, L, D)
+        t = torch.empty(((L - 1) << 25) + D, device="cuda").as_strided((1, 1, L, D), (0, 0, 1 << 25, 1))
+        t.copy_(randn(1, 1, L, D, seed=seed))
+        return t.expand(B, H, L, D)
+
+    if layout == "wide":
+        L = 9  # 1 GiB of rows
+    q, k, v = (view(9830 + i) for i in range(3))
+    copies = [x.clone(memory_format=torch.contiguous_format) for x in (q, k, v)]
+    out = sdpa(q, k, v)
+    assert_bitwise(out, sdpa(*copies), "copy")
+    assert_bitwise(sdpa(q[1:2], k[1:2], v[1:2]), out[1:2], "one sample")
