@@ -54,6 +54,7 @@ struct F32AttnArgs {
   float scale;
   int32_t causal;
   int32_t mvec;  // mask rows have unit stride
+  int64_t tile0;   // first tile of the launch
   int32_t chunks;  // split launch: chunks of the longest key range
   float* partial;  // split launch: O^T of [chunk][pair][row][dv], then {m, l} of [chunk][pair][row]
   float* stats;
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
   __shared__ __attribute__((aligned(16))) char smem[2 * (K_BYTES + V_BYTES)];
 
   // longest causal key ranges first, all (batch, head) pairs per level
-  const int64_t t = SPLIT ? blockIdx.x / a.chunks : blockIdx.x;
+  const int64_t t = SPLIT ? blockIdx.x / a.chunks : a.tile0 + blockIdx.x;
   const int chunk0 = SPLIT ? (int)(blockIdx.x % a.chunks) : 0;
   const int qt = a.qtiles - 1 - (int)(t / a.pairs);
   const int64_t pair = t % a.pairs;
@@ -408,13 +409,22 @@ __global__ __launch_bounds__(256) void f32_combine_kernel(F32AttnArgs a) {
   *reinterpret_cast<f32x4_t*>(a.out + r * a.dv + col) = f32_final(o, m, l);
 }
 
+// Workgroups of a launch: fewer than 2^32 threads.  A call of more tiles (millions of samples of one
+// query row) takes several launches.
+constexpr int64_t kF32MaxGrid = ((int64_t(1) << 32) - 1) / 256;
+
 template <int DP, int QP, int DVP, bool SPLIT>
-static int launch_f32_masks(const F32AttnArgs& a, int mask_kind, hipStream_t s) {
-  const dim3 grid((unsigned)(a.pairs * a.qtiles * (SPLIT ? a.chunks : 1))), block(256);
-  if (mask_kind == 0) hipLaunchKernelGGL((f32_attn_kernel<DP, QP, DVP, 0, SPLIT>), grid, block, 0, s, a);
-  else if (mask_kind == 1) hipLaunchKernelGGL((f32_attn_kernel<DP, QP, DVP, 1, SPLIT>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((f32_attn_kernel<DP, QP, DVP, 2, SPLIT>), grid, block, 0, s, a);
-  return check_launch("f32_attn_kernel");
+static int launch_f32_masks(F32AttnArgs a, int mask_kind, hipStream_t s) {
+  const int64_t total = a.pairs * a.qtiles * (SPLIT ? a.chunks : 1);  // split: within one launch
+  for (a.tile0 = 0; a.tile0 < total; a.tile0 += kF32MaxGrid) {
+    const dim3 grid((unsigned)std::min(total - a.tile0, kF32MaxGrid)), block(256);
+    if (mask_kind == 0) hipLaunchKernelGGL((f32_attn_kernel<DP, QP, DVP, 0, SPLIT>), grid, block, 0, s, a);
+    else if (mask_kind == 1) hipLaunchKernelGGL((f32_attn_kernel<DP, QP, DVP, 1, SPLIT>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((f32_attn_kernel<DP, QP, DVP, 2, SPLIT>), grid, block, 0, s, a);
+    const int rc = check_launch("f32_attn_kernel");
+    if (rc != BIOPS_OK) return rc;
+  }
+  return BIOPS_OK;
 }
 template <int DP, int QP, int DVP>
 static int launch_f32_attn(const F32AttnArgs& a, int mask_kind, hipStream_t s) {
@@ -433,7 +443,7 @@ static int launch_f32_attn(const F32AttnArgs& a, int mask_kind, hipStream_t s) {
 static int64_t f32_split_chunks(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t dv) {
   const int64_t tiles = batch * hq * cdiv(lq, kF32Rows), chunks = cdiv(lk, kF32Chunk);
   if (chunks < 2 || tiles >= (chunks == 2 ? 1 : 2) * (int64_t)device_cus()) return 0;
-  if (tiles * chunks >= (int64_t(1) << 31) || cdiv(batch * hq * lq * (dv / 4), 256) >= (int64_t(1) << 31)) return 0;
+  if (tiles * chunks > kF32MaxGrid || cdiv(batch * hq * lq * (dv / 4), 256) > kF32MaxGrid) return 0;
   return chunks;
 }
 static int64_t f32_stats_offset(int64_t chunks, int64_t rows, int64_t dv) {
@@ -445,9 +455,10 @@ static int64_t f32_stats_offset(int64_t chunks, int64_t rows, int64_t dv) {
 using namespace biops;
 
 extern "C" int biops_sdpa_f32_supported(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t d, int64_t dv) {
-  const int64_t lim = int64_t(1) << 31;
-  return d >= 1 && d <= 128 && dv >= 1 && dv <= 128 && d % 4 == 0 && dv % 4 == 0 && lq < lim / 2 && lk < lim / 2 &&
-         batch * hq < lim && batch * hq * cdiv(lq, kF32Rows) < lim;
+  const int64_t lim = int64_t(1) << 30;  // the sizes of one sample: the path must not depend on the batch
+  (void)batch;
+  (void)hq;
+  return d >= 1 && d <= 128 && dv >= 1 && dv <= 128 && d % 4 == 0 && dv % 4 == 0 && lq < lim && lk < lim;
 }
 
 extern "C" int64_t biops_sdpa_f32_workspace_size(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t d, int64_t dv) {

@@ -27,6 +27,8 @@ def test_sizes_taken_and_argument_errors():
     ok = lib.biops_sdpa_f32_supported
     assert ok(2, 4, 7, 9, 4, 128) and ok(1, 1, 1, 0, 128, 4)
     assert not ok(1, 1, 1, 1, 132, 4) and not ok(1, 1, 1, 1, 6, 4) and not ok(1, 1, 1, 1, 4, 130)
+    for batch in (1, 1 << 24, 1 << 32):  # any number of samples: the path depends on one sample's sizes
+        assert ok(batch, 16, 1, 5, 64, 64) and lib.biops_sdpa_f32_workspace_size(batch, 16, 1, 500, 64, 64) >= 0
     p = 256
 
     def call(d=64, q=p, sk=64, hkv=2, mask=None, mcode=0, causal=0):
@@ -201,3 +203,15 @@ def test_f32_sdpa_views_give_the_bits_of_their_copies(layout):
     out = sdpa(q, k, v)
     assert_bitwise(out, sdpa(*copies), "copy")
     assert_bitwise(sdpa(q[1:2], k[1:2], v[1:2]), out[1:2], "one sample")
+
+
+@pytest.mark.gpu
+def test_f32_sdpa_of_more_tiles_than_a_launch_has():
+    """2^24 and some query tiles: 256 threads each are more than one launch takes."""
+    B, H = (1 << 20) + 3, 16
+    q = torch.randn(B, H, 1, 4, generator=torch.Generator("cuda").manual_seed(9840), device="cuda")
+    k, v = (randn(1, H, 5, 4, seed=9841 + i).cuda() for i in range(2))
+    out = sdpa(q, k.expand(B, H, 5, 4), v.expand(B, H, 5, 4))
+    for rows in (slice(0, 2), slice(B - 5, B)):
+        n = rows.stop - rows.start
+        assert_bitwise(sdpa(q[rows], k.expand(n, H, 5, 4), v.expand(n, H, 5, 4)), out[rows], str(rows))
