@@ -74,12 +74,9 @@ __device__ __forceinline__ float f32_exp(float x, float m) {
   return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(a), (int)e);
 }
 
-// False for a chunk without a visible key.  A chunk whose scores are all NaN has the maximum -inf too,
-// but a NaN sum.
-__device__ __forceinline__ bool f32_any(float m, float l) { return m != -INFINITY || l != 0.f; }
-
-// Adds a chunk's (mc, lc) with at least one visible key to the running (m, l); the running O becomes
-// O * c1 + Oc * c2 (f32_merge_o).
+// Adds a chunk's (mc, lc) to the running (m, l); the running O becomes O * c1 + Oc * c2 (f32_merge_o).
+// A chunk whose keys are all masked is added too, with the weight 0 that its keys have: what its
+// values hold (NaN, infinities) reaches the row, as in the composite's product.
 __device__ __forceinline__ void f32_merge(float& m, float& l, float mc, float lc, float& c1, float& c2) {
   const float mn = fmaxf(m, mc);
   c1 = m == mn ? 1.f : f32_exp(m, mn);
@@ -330,7 +327,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
       return;
     }
     // the last chunk's merge divides by the row sum and stores the result
-    const bool first = mt == -INFINITY, some = f32_any(m, lc);
+    const bool first = chunk == 0, some = chunk * kF32Chunk < lim;  // rows that end before the chunk have none of it
     if (row_ok && (some || last)) {
       float c1 = 1.f, c2 = 0.f;
       if (some) f32_merge(mt, lt, m, lc, c1, c2);
@@ -341,7 +338,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
         for (int j = 0; j < 4; ++j) {
           const int col = 32 * e + 8 * j + 4 * hf;
           o[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-          if (!first) o[j] = *reinterpret_cast<const f32x4_t*>(orow + (col < a.dv ? col : 0));
+          if (!first && lim > 0) o[j] = *reinterpret_cast<const f32x4_t*>(orow + (col < a.dv ? col : 0));
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -399,12 +396,10 @@ __global__ __launch_bounds__(256) void f32_combine_kernel(F32AttnArgs a) {
   for (int c = 0; c < nc; ++c) {
     const f32x2_t st = *reinterpret_cast<const f32x2_t*>(a.stats + 2 * (c * rows + r));
     const f32x4_t oc = *reinterpret_cast<const f32x4_t*>(a.partial + (c * rows + r) * a.dv + col);
-    if (!f32_any(st[0], st[1])) continue;
-    const bool first = m == -INFINITY;
     float c1, c2;
     f32_merge(m, l, st[0], st[1], c1, c2);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = f32_merge_o(o[e], oc[e], c1, c2, first);
+    for (int e = 0; e < 4; ++e) o[e] = f32_merge_o(o[e], oc[e], c1, c2, c == 0);
   }
   *reinterpret_cast<f32x4_t*>(a.out + r * a.dv + col) = f32_final(o, m, l);
 }

@@ -215,3 +215,23 @@ def test_f32_sdpa_of_more_tiles_than_a_launch_has():
     for rows in (slice(0, 2), slice(B - 5, B)):
         n = rows.stop - rows.start
         assert_bitwise(sdpa(q[rows], k.expand(n, H, 5, 4), v.expand(n, H, 5, 4)), out[rows], str(rows))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", (1, 160))
+def test_f32_sdpa_values_behind_a_mask(B, monkeypatch):
+    """A masked key has the weight 0, and 0 times NaN or infinity is NaN in every row that attends to anything:
+    in the 128 keys of a chunk without a visible key as elsewhere."""
+    q, k, v = (randn(B, 4, 400, 64, seed=9850 + i).cuda() for i in range(3))
+    mask = torch.ones(B, 1, 1, 400, dtype=torch.bool, device="cuda")
+    mask[..., :150] = False
+    mask[..., 260:] = False
+    v[:, 0, 3, 5] = math.nan
+    v[:, 1, 130, 6] = math.inf
+    v[:, 2, 390, 7] = math.nan
+    out = sdpa(q, k, v, attn_mask=mask)
+    for head, column in ((0, 5), (1, 6), (2, 7)):
+        assert out[:, head, :, column].isnan().all()
+    assert int(out.isnan().sum()) == 3 * B * 400
+    monkeypatch.setenv("BIOPS_ATTENTION_MATERIALIZE", "1")
+    assert torch.equal(sdpa(q, k, v, attn_mask=mask).isnan(), out.isnan())
