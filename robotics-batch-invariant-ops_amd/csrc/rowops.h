@@ -105,28 +105,33 @@ __device__ __forceinline__ void store_row_chunk(T* row, int64_t cols, int64_t c0
 // exp(x - m) for the softmax family, m the row's maximum (or 0 for a row of -inf): the accurate libm
 // expf when the result is stored as fp32; when it is rounded to 16 bits anyway, the hardware exp2
 // of fma(x, log2 e, -m log2 e).  The rounding of m log2 e is common to the row and cancels in the
-// division by the row sum while it is small; a row whose maximum is huge (masked with the type's
-// lowest value, where the product overflows) takes the difference first instead.
+// division by the row sum while it is small, but not for a row whose maximum is huge (masked with
+// the type's lowest value, where the product overflows).  From |m| = 2^16 on, bf16 rows therefore
+// use exp2(x - m), exact: neighbouring bf16 values differ by 2^8 and more there, so every term is 1
+// or 0 either way (fp16 ends at 65504); fp32 rows take the difference first, in a branch of their
+// own (tested for in every row, it cost the bf16 ones 4 %).
 constexpr float kLog2e = 1.4426950408889634f;
 struct SoftShift {
-  float m, ml2e;
-  bool wide;  // |m log2 e| >= 2^16 (its rounding is 2^-8 and more), the same in the whole wavefront
+  float m, k, sh;  // exp(x - m) = exp2(x * k - sh)
+  bool wide;       // fp32 rows: |m| >= 2^16, the same in the whole wavefront
 };
+template <typename Tin>
 __device__ __forceinline__ SoftShift soft_shift(float m) {
-  const float ml2e = m * kLog2e;
-  return SoftShift{m, ml2e, (bool)__any(fabsf(ml2e) >= 65536.f)};
+  const bool huge = fabsf(m) >= 65536.f;
+  if constexpr (std::is_same<Tin, bf16_t>::value) return SoftShift{m, huge ? 1.f : kLog2e, huge ? m : m * kLog2e, false};
+  return SoftShift{m, kLog2e, m * kLog2e, sizeof(Tin) == 4 && __any(huge)};
 }
-template <typename Tout, int N>
+template <typename Tin, typename Tout, int N>
 __device__ __forceinline__ void soft_exp(float (&v)[N], const SoftShift& s) {
   if constexpr (sizeof(Tout) == 4) {
 #pragma unroll
     for (int e = 0; e < N; ++e) v[e] = expf(v[e] - s.m);
-  } else if (__builtin_expect(s.wide, 0)) {
+  } else if (sizeof(Tin) == 4 && __builtin_expect(s.wide, 0)) {
 #pragma unroll
     for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f((v[e] - s.m) * kLog2e);
   } else {
 #pragma unroll
-    for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[e], kLog2e, -s.ml2e));
+    for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[e], s.k, -s.sh));
   }
 }
 
@@ -197,7 +202,7 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
   }
   mx = wave_max(mx);
   const bool all_neg_inf = (mx == -INFINITY);
-  const SoftShift shift = soft_shift(all_neg_inf ? 0.f : mx);
+  const SoftShift shift = soft_shift<T>(all_neg_inf ? 0.f : mx);
 
   float sum = 0.f;
   if (fits) {
@@ -205,7 +210,7 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
     for (int j = 0; j < kRowRegChunks; ++j) {
       const int64_t ci = lane + 64 * j;
       if (ci < nchunks) {
-        soft_exp<T>(cache[j], shift);
+        soft_exp<T, T>(cache[j], shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           if (all_neg_inf) cache[j][e] = 0.f;
@@ -218,7 +223,7 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
       float v[VEC];
       load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
       transform_chunk<T>(ar, ci * VEC, cols, v);
-      soft_exp<T>(v, shift);
+      soft_exp<T, T>(v, shift);
 #pragma unroll
       for (int e = 0; e < VEC; ++e)
         if (ci * VEC + e < cols) sum += all_neg_inf ? 0.f : v[e];
@@ -244,7 +249,7 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
       float v[VEC];
       load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
       transform_chunk<T>(ar, ci * VEC, cols, v);
-      soft_exp<T>(v, shift);
+      soft_exp<T, T>(v, shift);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) v[e] = zero || all_neg_inf ? 0.f : v[e] * inv;
       store_row_chunk<T, VEC>(row, cols, ci * VEC, v);
@@ -297,7 +302,7 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     neg_inf[r] = (mx[r] == -INFINITY);
-    const SoftShift shift = soft_shift((MODE == kLogSoftmax || !neg_inf[r]) ? mx[r] : 0.f);
+    const SoftShift shift = soft_shift<Tin>((MODE == kLogSoftmax || !neg_inf[r]) ? mx[r] : 0.f);
     sum[r] = 0.f;
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
@@ -306,7 +311,7 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
         float ex[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) ex[e] = cache[r][j][e];
-        soft_exp<Tout>(ex, shift);
+        soft_exp<Tin, Tout>(ex, shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           if (MODE != kLogSoftmax) cache[r][j][e] = ex[e] = neg_inf[r] ? 0.f : ex[e];

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
   };
   // exp of a column past the row end is 0 (NaN only where the whole row gives NaN)
   auto exps = [&](float (&v)[VEC], bool neg_inf, const SoftShift& shift) {
-    soft_exp<Tout>(v, shift);
+    soft_exp<Tin, Tout>(v, shift);
     if (MODE != kLogSoftmax && neg_inf) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) v[e] = 0.f;
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
   mx = block_max<NW>(mx, part[0]);
   keep_raw();
   const bool neg_inf = (mx == -INFINITY);
-  const SoftShift shift = soft_shift((MODE == kLogSoftmax || !neg_inf) ? mx : 0.f);
+  const SoftShift shift = soft_shift<Tin>((MODE == kLogSoftmax || !neg_inf) ? mx : 0.f);
 
   // fp32 softmax of a resident row keeps the exponentials in the row's registers
   constexpr bool kKeepExp = !LOOP && sizeof(Tin) == 4 && MODE == kSoftmax;
