@@ -1,4 +1,5 @@
 // Softmax / log-softmax and mean / L2-norm reductions.
+#include <algorithm>
 #include <type_traits>
 
 #include "rowops.h"
@@ -179,25 +180,52 @@ __global__ __launch_bounds__(256) void softmax_fit_kernel(SoftmaxArgs a) {
                                            a.cols);
 }
 
+// A launch has fewer than 2^32 threads: rows beyond that go to further launches of the same kernel.
+// Calls launch(first row, rows) with at most `per_group` rows per `threads` threads.
+template <typename F>
+static int launch_row_ranges(int64_t rows, int per_group, int threads, F&& launch) {
+  const int64_t most = ((int64_t(1) << 32) - 1) / threads * per_group;
+  for (int64_t first = 0; first < rows; first += most) {
+    const int rc = launch(first, std::min(rows - first, most));
+    if (rc != BIOPS_OK) return rc;
+  }
+  return BIOPS_OK;
+}
+
+template <typename Tin, typename Tout>
+static SoftmaxArgs softmax_rows_from(const SoftmaxArgs& a, int64_t first, int64_t rows) {
+  SoftmaxArgs b = a;
+  b.in = reinterpret_cast<const Tin*>(a.in) + first * a.ld_in;
+  b.out = reinterpret_cast<Tout*>(a.out) + first * a.ld_out;
+  b.rows = rows;
+  return b;
+}
+
 template <typename Tin, typename Tout, int NC>
 static int launch_softmax_fit(const SoftmaxArgs& a, int is_log, hipStream_t s) {
-  const int64_t blocks = cdiv(a.rows, kRowWaves * fit_rows<NC>());
-  if (blocks > 0x7fffffffLL) return fail(BIOPS_ERR_ARG, "too many rows");
-  if (is_log)
-    hipLaunchKernelGGL((softmax_fit_kernel<Tin, Tout, kLogSoftmax, NC>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((softmax_fit_kernel<Tin, Tout, kSoftmax, NC>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  return check_launch("softmax_fit_kernel");
+  constexpr int kRows = kRowWaves * fit_rows<NC>();
+  return launch_row_ranges(a.rows, kRows, 256, [&](int64_t first, int64_t rows) {
+    const SoftmaxArgs b = softmax_rows_from<Tin, Tout>(a, first, rows);
+    const dim3 grid((unsigned)cdiv(rows, kRows));
+    if (is_log)
+      hipLaunchKernelGGL((softmax_fit_kernel<Tin, Tout, kLogSoftmax, NC>), grid, dim3(256), 0, s, b);
+    else
+      hipLaunchKernelGGL((softmax_fit_kernel<Tin, Tout, kSoftmax, NC>), grid, dim3(256), 0, s, b);
+    return check_launch("softmax_fit_kernel");
+  });
 }
 
 template <typename Tin, typename Tout, int T, int NC, bool LOOP = false>
 static int launch_softmax_block(const SoftmaxArgs& a, int is_log, hipStream_t s) {
-  if (a.rows > 0x7fffffffLL) return fail(BIOPS_ERR_ARG, "too many rows");
-  if (is_log)
-    hipLaunchKernelGGL((softmax_block_kernel<Tin, Tout, kLogSoftmax, T, NC, LOOP>), dim3((unsigned)a.rows), dim3(T), 0, s, a);
-  else
-    hipLaunchKernelGGL((softmax_block_kernel<Tin, Tout, kSoftmax, T, NC, LOOP>), dim3((unsigned)a.rows), dim3(T), 0, s, a);
-  return check_launch("softmax_block_kernel");
+  return launch_row_ranges(a.rows, 1, T, [&](int64_t first, int64_t rows) {
+    const SoftmaxArgs b = softmax_rows_from<Tin, Tout>(a, first, rows);
+    const dim3 grid((unsigned)rows);
+    if (is_log)
+      hipLaunchKernelGGL((softmax_block_kernel<Tin, Tout, kLogSoftmax, T, NC, LOOP>), grid, dim3(T), 0, s, b);
+    else
+      hipLaunchKernelGGL((softmax_block_kernel<Tin, Tout, kSoftmax, T, NC, LOOP>), grid, dim3(T), 0, s, b);
+    return check_launch("softmax_block_kernel");
+  });
 }
 
 template <typename Tin, typename Tout>
@@ -415,23 +443,36 @@ __global__ __launch_bounds__(256) void reduce_strided(ReduceArgs a) {
 }
 
 template <typename Tin, typename Tout, int OP>
+static int launch_reduce_rows(const ReduceArgs& a0, hipStream_t s) {
+  constexpr int VEC = 16 / (int)sizeof(Tin);
+  const int64_t nc = cdiv(cdiv(a0.N, VEC), 64);  // chunks per lane
+  const bool wave = nc <= kWaveRowChunks / 64, narrow = nc <= kBlock256Chunks / 64;
+  return launch_row_ranges(a0.M, wave ? kRowWaves : 1, narrow ? 256 : 1024, [&](int64_t first, int64_t rows) {
+    ReduceArgs a = a0;
+    a.in = reinterpret_cast<const Tin*>(a0.in) + first * a0.sM;
+    a.out = reinterpret_cast<Tout*>(a0.out) + first;
+    a.M = rows;
+    const dim3 grid((unsigned)(wave ? cdiv(rows, kRowWaves) : rows));
+    if (wave && a.N % VEC == 0) {
+      if (nc <= 1) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 1>), grid, dim3(256), 0, s, a);
+      else if (nc <= 2) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 2>), grid, dim3(256), 0, s, a);
+      else if (nc <= 4) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 4>), grid, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 8>), grid, dim3(256), 0, s, a);
+    } else if (wave) {
+      hipLaunchKernelGGL((reduce_rows_wave<Tin, Tout, OP>), grid, dim3(256), 0, s, a);
+    } else if (narrow) {
+      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP, 256>), grid, dim3(256), 0, s, a);
+    } else {
+      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP, 1024>), grid, dim3(1024), 0, s, a);
+    }
+    return check_launch("reduce");
+  });
+}
+
+template <typename Tin, typename Tout, int OP>
 static int launch_reduce(const ReduceArgs& a, hipStream_t s) {
   if (a.K == 1) {
-    constexpr int VEC = 16 / (int)sizeof(Tin);
-    const int64_t blocks = cdiv(a.M, kRowWaves);
-    const int64_t nc = cdiv(cdiv(a.N, VEC), 64);  // chunks per lane
-    if (a.N % VEC == 0 && nc <= kWaveRowChunks / 64) {
-      if (nc <= 1) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 1>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-      else if (nc <= 2) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 2>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-      else if (nc <= 4) hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 4>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((reduce_rows_fit<Tin, Tout, OP, 8>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-    } else if (nc <= kWaveRowChunks / 64) {
-      hipLaunchKernelGGL((reduce_rows_wave<Tin, Tout, OP>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-    } else if (nc <= kBlock256Chunks / 64) {
-      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP, 256>), dim3((unsigned)a.M), dim3(256), 0, s, a);
-    } else {
-      hipLaunchKernelGGL((reduce_rows_block<Tin, Tout, OP, 1024>), dim3((unsigned)a.M), dim3(1024), 0, s, a);
-    }
+    return launch_reduce_rows<Tin, Tout, OP>(a, s);
   } else if (a.kvec) {
     constexpr int VK = 16 / (int)sizeof(Tin);
     const int64_t blocks = a.M * cdiv(a.K, 64 * VK);

@@ -15,6 +15,7 @@ from batch_invariant_ops import (
     set_batch_invariant_mode,
     softmax,
 )
+from batch_invariant_ops import _native as nat
 
 from _tol import assert_bitwise, assert_close_scaled, assert_first_sample_equal
 
@@ -227,3 +228,25 @@ def test_softmax_rows_of_the_lowest_value(dtype_in, dtype_out, cols):
         ref = torch.log_softmax(x.double(), -1)
         # x - max - log(sum): the two roundings of a bf16 output's fp32 value and the output's own
         assert torch.allclose(logp.double(), ref, rtol=2.0**-8 if dtype_in == torch.bfloat16 else 2.0**-20)
+
+
+# Long rows have a workgroup each, and a launch ends at 2^32 threads: 2^24 workgroups of 256, 2^22 of
+# 1024.  The rows here are one row of memory (row stride 0).
+@pytest.mark.parametrize("rows,cols", (((1 << 24) + 5, 4104), ((1 << 22) + 5, 16392)))
+def test_reduction_of_more_rows_than_a_launch_has(rows, cols):
+    x = randn(1, cols, seed=880, dtype=torch.bfloat16).cuda()
+    out = torch.full((rows,), math.nan, dtype=torch.bfloat16, device="cuda")
+    nat.call("biops_reduce", nat.REDUCE_MEAN, nat.BF16, nat.BF16, rows, cols, 1, x.data_ptr(), 0, 1, 1, out.data_ptr(),
+             nat.stream_of(out))
+    assert bool((out == mean_dim(x, -1)).all())
+
+
+@pytest.mark.parametrize("rows,cols", (((1 << 24) + 5, 1028), ((1 << 22) + 5, 4100)))
+def test_softmax_of_more_rows_than_a_launch_has(rows, cols):
+    x = randn(1, cols, seed=881).cuda()
+    out = torch.empty(rows, cols, dtype=torch.float16, device="cuda")  # 34 GB
+    out[-6:] = math.nan
+    nat.call("biops_softmax", nat.F32, nat.F16, rows, cols, x.data_ptr(), 0, out.data_ptr(), cols, 0, nat.stream_of(out))
+    row = softmax(x, -1, dtype=torch.float16)
+    for part in out.split(1 << 20):
+        assert bool((part == row).all())
