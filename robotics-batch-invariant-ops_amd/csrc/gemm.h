@@ -6,7 +6,8 @@
 
 namespace biops {
 
-enum { kEpiPlain = 0, kEpiBias = 1, kEpiSwiglu = 2 };
+// kEpiRowBias: kernels with BmmArgs::row_bias (launch_bmm takes kEpiPlain and picks them).
+enum { kEpiPlain = 0, kEpiBias = 1, kEpiSwiglu = 2, kEpiRowBias = 3 };
 
 // One launch covers nb1*nb2 independent GEMMs C[b] = A[b] . B[b] of equal shape.
 // Batch b = b1*nb2 + b2 addresses X + b1*sX1 + (b2/gX)*sX2 (gA = gC = 1, gB = args.gB).

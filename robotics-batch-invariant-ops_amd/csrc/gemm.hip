@@ -153,7 +153,7 @@ __device__ __forceinline__ void bmm_tile(const BmmArgs& args, uint32_t t, char* 
   src.p0 = reinterpret_cast<const T*>(args.B) + boff;
   src.p1 = EPI == kEpiSwiglu ? reinterpret_cast<const T*>(args.B2) + boff : src.p0;
   src.ld = args.ldb;
-  src.ncols = args.N - n0 + (BKM || GRP ? 0 : args.b_extra);
+  src.ncols = args.N - n0 + (BKM || GRP || !DIRECT ? 0 : args.b_extra);
   src.swiglu = EPI == kEpiSwiglu;
   src.vec_ok = args.b_vec != 0;
   const int64_t rows = o.m_end - m0;
@@ -173,13 +173,12 @@ __device__ __forceinline__ void bmm_tile(const BmmArgs& args, uint32_t t, char* 
   }
 
   T* Cp = reinterpret_cast<T*>(args.C) + b1 * args.sC1 + b2 * args.sC2 + m0 * args.ldc + n0;
-  constexpr bool kRowBias = EPI == kEpiPlain && BKM && !GRP;
-  const T* bias = nullptr;
-  const T* row_bias = nullptr;
-  if (EPI != kEpiSwiglu && args.bias) {
-    if (kRowBias && args.row_bias) row_bias = reinterpret_cast<const T*>(args.bias) + b2 * args.M + m0;
-    else bias = reinterpret_cast<const T*>(args.bias) + n0;
-  }
+  // A row bias has kernels of its own: a test for one at run time cost the bias-free products 1 % (2 x 568 ->
+  // 2995, fp16, 10.67 -> 10.76 us per test in the store loop, 10.83 per tile).
+  constexpr bool kRowBias = EPI == kEpiRowBias;
+  static_assert(!kRowBias || (BKM && !GRP), "row bias: K-major B, no row groups");
+  const T* bias = (EPI != kEpiSwiglu && !kRowBias && args.bias) ? reinterpret_cast<const T*>(args.bias) + n0 : nullptr;
+  const T* row_bias = kRowBias ? reinterpret_cast<const T*>(args.bias) + b2 * args.M + m0 : nullptr;
   Tile::template epilogue<EPI == kEpiSwiglu, kRowBias>(smem, acc, Cp, args.ldc, rows < BM ? (int)rows : BM,
                                                        cols < kCols ? (int)cols : kCols, bias, row_bias,
                                                        args.c_vec != 0);
@@ -783,6 +782,30 @@ static int launch_typed(const BmmArgs& a, bool b_kmajor, bool direct, int cfg, h
   }
 }
 
+// Row bias: K-major B.  Without direct loads (BIOPS_GEMM_NO_DIRECT only: a convolution's operands are
+// aligned) one entry is enough, all entries giving the same bits.
+template <typename T>
+static int launch_row_bias(const BmmArgs& a, bool direct, int cfg, hipStream_t s) {
+  if (cfg == kSkinnyCfg) return launch_skinny<T>(a, s);
+  if (!direct) return launch_cfg<T, 2, true, false, kEpiRowBias, false>(a, s);
+  switch (cfg) {
+    case 0: if constexpr (sizeof(T) == 2) return launch_cfg<T, 0, true, true, kEpiRowBias, false>(a, s); break;
+    case 1: return launch_cfg<T, 1, true, true, kEpiRowBias, false>(a, s);
+    case 2: return launch_cfg<T, 2, true, true, kEpiRowBias, false>(a, s);
+    case 3: return launch_cfg<T, 3, true, true, kEpiRowBias, false>(a, s);
+    case 4: return launch_cfg<T, 4, true, true, kEpiRowBias, false>(a, s);
+    case 5: return launch_cfg<T, 5, true, true, kEpiRowBias, false>(a, s);
+    case 6: return launch_cfg<T, 6, true, true, kEpiRowBias, false>(a, s);
+    case 7: return launch_cfg<T, 7, true, true, kEpiRowBias, false>(a, s);
+    case 8: return launch_cfg<T, 8, true, true, kEpiRowBias, false>(a, s);
+    case 9: if constexpr (sizeof(T) == 2) return launch_cfg<T, 9, true, true, kEpiRowBias, false>(a, s); break;
+    case 10: return launch_cfg<T, 10, true, true, kEpiRowBias, false>(a, s);
+    case 11: return launch_cfg<T, 11, true, true, kEpiRowBias, false>(a, s);
+    default: break;
+  }
+  return fail(BIOPS_ERR_ARG, "no row-bias kernel for tile config %d", cfg);
+}
+
 // BIOPS_GEMM_NO_DIRECT (any value) forces the register load path (read once per process).
 static bool direct_disabled() {
   static const bool off = getenv("BIOPS_GEMM_NO_DIRECT") != nullptr;
@@ -874,6 +897,15 @@ int launch_bmm(int dtype, BmmArgs a, int epi, bool b_kmajor, hipStream_t stream)
                                  : launch_grouped_typed<bf16_t, kEpiPlain>(a, b_kmajor, direct, cfg, stream);
       default:
         return fail(BIOPS_ERR_DTYPE, "unsupported GEMM dtype %d", dtype);
+    }
+  }
+  if (a.row_bias) {
+    if (epi != kEpiPlain || !b_kmajor || !a.bias) return fail(BIOPS_ERR_ARG, "row bias: plain products with a K-major B");
+    switch (dtype) {
+      case BIOPS_F32: return launch_row_bias<float>(a, direct, cfg, stream);
+      case BIOPS_F16: return launch_row_bias<f16_t>(a, direct, cfg, stream);
+      case BIOPS_BF16: return launch_row_bias<bf16_t>(a, direct, cfg, stream);
+      default: return fail(BIOPS_ERR_DTYPE, "unsupported GEMM dtype %d", dtype);
     }
   }
   switch (dtype) {

@@ -704,7 +704,7 @@ struct GemmTile {
   // blocks (i, j) / (i, j+1) of the same lane; the stored value is
   // round(round(silu(round(g))) * round(u)) and the tile is BN/2 wide.  Otherwise the value is
   // round(acc + bias[col]) (bias may be null: no add), and with ROWB the written value is
-  // round(that + row_bias[row]) (row_bias may be null).  Ends with a barrier, so the LDS ring is free for the next tile.
+  // round(that + row_bias[row]).  Ends with a barrier, so the LDS ring is free for the next tile.
   template <bool SWIGLU, bool ROWB = false>
   __device__ static __forceinline__ void epilogue(char* smem, Acc (&acc)[FM][FN], T* C,
                                                   int64_t ldc, int rows, int cols, const T* bias,
@@ -744,17 +744,15 @@ struct GemmTile {
       const char* src = smem + r * PITCH + (((c0 / VEC) ^ (r & SWZ)) * 16);
       T* dst = C + (int64_t)r * ldc + c0;
       if constexpr (ROWB) {
-        if (row_bias) {
-          const u32x4_t v = add_round<T>(*reinterpret_cast<const u32x4_t*>(src), Num<T>::load(row_bias + r));
-          if (c_vec && c0 + VEC <= cols) {
-            *reinterpret_cast<u32x4_t*>(dst) = v;
-          } else {
+        const u32x4_t v = add_round<T>(*reinterpret_cast<const u32x4_t*>(src), Num<T>::load(row_bias + r));
+        if (c_vec && c0 + VEC <= cols) {
+          *reinterpret_cast<u32x4_t*>(dst) = v;
+        } else {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e)
-              if (c0 + e < cols) dst[e] = reinterpret_cast<const T*>(&v)[e];
-          }
-          continue;
+          for (int e = 0; e < VEC; ++e)
+            if (c0 + e < cols) dst[e] = reinterpret_cast<const T*>(&v)[e];
         }
+        continue;
       }
       if (c_vec && c0 + VEC <= cols) {
         *reinterpret_cast<u32x4_t*>(dst) = *reinterpret_cast<const u32x4_t*>(src);
