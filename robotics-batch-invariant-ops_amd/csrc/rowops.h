@@ -121,18 +121,11 @@ __device__ __forceinline__ SoftShift soft_shift(float m) {
   if constexpr (std::is_same<Tin, bf16_t>::value) return SoftShift{m, huge ? 1.f : kLog2e, huge ? m : m * kLog2e, false};
   return SoftShift{m, kLog2e, m * kLog2e, sizeof(Tin) == 4 && __any(huge)};
 }
-template <typename Tin, typename Tout, int N>
-__device__ __forceinline__ void soft_exp(float (&v)[N], const SoftShift& s) {
-  if constexpr (sizeof(Tout) == 4) {
-#pragma unroll
-    for (int e = 0; e < N; ++e) v[e] = expf(v[e] - s.m);
-  } else if (sizeof(Tin) == 4 && __builtin_expect(s.wide, 0)) {
-#pragma unroll
-    for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f((v[e] - s.m) * kLog2e);
-  } else {
-#pragma unroll
-    for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[e], s.k, -s.sh));
-  }
+template <typename Tin, typename Tout>
+__device__ __forceinline__ float soft_exp(float x, const SoftShift& s) {
+  if constexpr (sizeof(Tout) == 4) return expf(x - s.m);
+  if (sizeof(Tin) == 4 && __builtin_expect(s.wide, 0)) return __builtin_amdgcn_exp2f((x - s.m) * kLog2e);
+  return __builtin_amdgcn_exp2f(__builtin_fmaf(x, s.k, -s.sh));
 }
 
 // ------------------------------------------------------------------ softmax rows ----
@@ -210,10 +203,9 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
     for (int j = 0; j < kRowRegChunks; ++j) {
       const int64_t ci = lane + 64 * j;
       if (ci < nchunks) {
-        soft_exp<T, T>(cache[j], shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          if (all_neg_inf) cache[j][e] = 0.f;
+          cache[j][e] = all_neg_inf ? 0.f : soft_exp<T, T>(cache[j][e], shift);
           if (ci * VEC + e < cols) sum += cache[j][e];
         }
       }
@@ -223,10 +215,11 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
       float v[VEC];
       load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
       transform_chunk<T>(ar, ci * VEC, cols, v);
-      soft_exp<T, T>(v, shift);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e)
-        if (ci * VEC + e < cols) sum += all_neg_inf ? 0.f : v[e];
+      for (int e = 0; e < VEC; ++e) {
+        const float ex = all_neg_inf ? 0.f : soft_exp<T, T>(v[e], shift);
+        if (ci * VEC + e < cols) sum += ex;
+      }
     }
   }
   sum = wave_sum(sum);
@@ -249,10 +242,11 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
       float v[VEC];
       load_row_chunk<T>(row, cols, ci * VEC, -INFINITY, v);
       transform_chunk<T>(ar, ci * VEC, cols, v);
-      soft_exp<T, T>(v, shift);
+      float o[VEC];
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) v[e] = zero || all_neg_inf ? 0.f : v[e] * inv;
-      store_row_chunk<T, VEC>(row, cols, ci * VEC, v);
+      for (int e = 0; e < VEC; ++e)
+        o[e] = zero ? 0.f : (all_neg_inf ? 0.f : soft_exp<T, T>(v[e], shift)) * inv;
+      store_row_chunk<T, VEC>(row, cols, ci * VEC, o);
     }
   }
 }
@@ -308,14 +302,11 @@ __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, T
     for (int j = 0; j < NC; ++j) {
       const int64_t ci = lane + 64 * j;
       if (ci < nchunks) {
-        float ex[VEC];
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) ex[e] = cache[r][j][e];
-        soft_exp<Tin, Tout>(ex, shift);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          if (MODE != kLogSoftmax) cache[r][j][e] = ex[e] = neg_inf[r] ? 0.f : ex[e];
-          if (ci * VEC + e < cols) sum[r] += ex[e];
+          const float ex = (MODE != kLogSoftmax && neg_inf[r]) ? 0.f : soft_exp<Tin, Tout>(cache[r][j][e], shift);
+          if (MODE != kLogSoftmax) cache[r][j][e] = ex;
+          if (ci * VEC + e < cols) sum[r] += ex;
         }
       }
     }

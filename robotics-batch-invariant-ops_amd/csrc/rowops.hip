@@ -94,11 +94,9 @@ __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
   };
   // exp of a column past the row end is 0 (NaN only where the whole row gives NaN)
   auto exps = [&](float (&v)[VEC], bool neg_inf, const SoftShift& shift) {
-    soft_exp<Tin, Tout>(v, shift);
-    if (MODE != kLogSoftmax && neg_inf) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) v[e] = 0.f;
-    }
+    for (int e = 0; e < VEC; ++e)
+      v[e] = (MODE != kLogSoftmax && neg_inf) ? 0.f : soft_exp<Tin, Tout>(v[e], shift);
   };
 
   float mx = -INFINITY;
