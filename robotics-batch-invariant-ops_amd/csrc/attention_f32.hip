@@ -17,20 +17,20 @@
 // The keys are cut into chunks of kF32Chunk, each with its own maximum, sum and O^T, and the chunks
 // are merged in order (f32_merge): by the workgroup itself, which then keeps the running total in the
 // output rows, or, when the launch has too few query tiles to fill the chip, by f32_combine_kernel
-// after a launch with one workgroup per chunk.  Both do the same operations in the same order, so
-// the choice, which depends on the batch, changes no bit.
+// after a launch with one workgroup per chunk; the smallest launches have workgroups of 32 query
+// rows that share a chunk's blocks (f32_few_kernel).  All do the same operations in the same order,
+// so the choice, which depends on the batch, changes no bit.
 //
 // Batch invariance: the chunks, the block order, the MFMA chains and the statistics depend on the
 // sample's own rows and lengths only.
 //
 // Bound: the fp32 matrix rate (157 TF/s): 4 x 9 + 16 x 3 MFMAs of 64 cycles per 32 x 32 block at
-// head size 72, beside about 130 vector instructions.  MI355X, against scores in memory (three
-// launches): 8 x 16 heads x 256 x 256, head size 72 (2.4 GFLOP, 18 us at the matrix rate) 72 -> 41 us;
-// causal 2 x 8 / 2 heads x 1000 x 1000, 128: 143 -> 103; causal 4 x 32 / 8 x 1500 x 1500, 64: 1655 -> 428;
-// 4 x 32 / 8 x 1500 x 1900, 128: 2810 -> 2020.  Of the 41 us the two products take about 20, the block loads
-// and barriers 5, the chunk merge 4, the softmax 2.5, launch and first loads the rest.  Chunks of
-// 256 keys saved the merges of large launches (1850 us there) but doubled the chain of the small
-// ones (1 head x 65 x 600: 32 -> 55 us; scores in memory 40).
+// head size 72, beside about 230 vector instructions.  MI355X, call times against scores in memory
+// (three launches): 8 x 16 heads x 256 x 256, head size 72 (2.4 GFLOP, 18 us at the matrix rate) 66.3 ->
+// 39.3 us; causal 2 x 8 / 2 heads x 1000 x 1000, 128: 133 -> 97; 1 x 16 heads, causal, 1024 x 1024, 64: 91 -> 56;
+// 4 x 32 / 8 x 1500 x 1500, 128, additive mask: 2780 -> 2010.  Of the 39 us the two products take about 20,
+// the block loads and barriers 5, the chunk merge 4, the softmax 4, launch and first loads the rest.
+// Chunks of 256 keys saved the merges of large launches but doubled the chain of the small ones.
 #include <algorithm>
 
 #include "gemm.h"
@@ -375,6 +375,158 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves<D
   if (!SPLIT && nblk == 0) end_chunk(0, true);  // no visible key: zeros
 }
 
+// Launches of few query rows: a workgroup per 32 rows and chunk, with the bits of f32_attn_kernel.
+// There a wavefront walks its chunk's four blocks by itself, a chain of 4 x (4 QP + 16) dependent MFMAs
+// (head size 128: 14 us) that a small launch has nothing to overlap with.  Here wavefront w computes
+// the scores and probabilities of block w, with the running maximum from the four block maxima, and
+// columns 32 w .. 32 w + 31 of O^T over the four blocks: 4 QP + 64 MFMAs in a row.  K, V and Q go from
+// memory to the operand registers; only the probabilities pass through LDS.  One chunk: the result
+// is written at once.
+template <int QP, int OF, int MASK>
+__global__ __launch_bounds__(256) void f32_few_kernel(F32AttnArgs a) {
+  constexpr int CB = kF32Chunk / kF32Keys;
+  static_assert(CB == 4 && OF <= 4, "a wavefront per block and per column block");
+  __shared__ float ps[CB][16][64], parts[CB][64], block_max[CB][32];
+  const int64_t t = blockIdx.x / a.chunks;
+  const int chunk = (int)(blockIdx.x % a.chunks);
+  const int qt = (int)((a.lq + 31) / 32 - 1 - t / a.pairs);
+  const int64_t pair = t % a.pairs;
+  const int64_t b = pair / a.hq, h = pair % a.hq, hk = h / a.group;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, hf = lane >> 5, l32 = lane & 31;
+  const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+  const int i0 = 32 * qt;
+  const int qrows = a.lq - i0 < 32 ? a.lq - i0 : 32;
+  const int shift = a.causal == BIOPS_CAUSAL_BOTTOM_RIGHT ? a.lk - a.lq : 0;
+  auto row_lim = [&](int r) -> int {
+    if (a.causal == BIOPS_CAUSAL_NONE) return a.lk;
+    const int c = i0 + r + shift + 1;
+    return c < 0 ? 0 : (c > a.lk ? a.lk : c);
+  };
+  const bool row_ok = l32 < qrows;
+  const int lim = row_ok ? row_lim(l32) : 0;
+  const int kend = row_lim(qrows - 1);
+  const int n0 = kF32Chunk * chunk;
+  if (chunk > 0 && n0 >= kend) return;  // no row has keys here
+
+  // V^T of column block w: register 16 j + r is key n0 + 32 j + 8(r/4) + 4 hf + r%4 (keys past the end read
+  // row 0 and are zeroed below)
+  float xv[CB][16];
+  if (w < OF) {
+    const float* const vb = a.v + b * a.svB + hk * a.svH + (32 * w + l32 < a.dv ? 32 * w + l32 : 0);
+#pragma unroll
+    for (int j = 0; j < CB; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int n = n0 + 32 * j + 8 * (r >> 2) + 4 * hf + (r & 3);
+        xv[j][r] = a.lk > 0 ? vb[(int64_t)(n < a.lk ? n : 0) * a.svL] : 0.f;
+      }
+  }
+  const int nw = n0 + 32 * w;  // this wavefront's block of keys
+  float s[16];
+  float bm = -INFINITY;
+  if (nw < kend) {
+    const float* const qr = a.q + b * a.sqB + h * a.sqH + (int64_t)(i0 + (row_ok ? l32 : 0)) * a.sqL;
+    const float* const kr = a.k + b * a.skB + hk * a.skH + (int64_t)(nw + l32 < a.lk ? nw + l32 : 0) * a.skL;
+    u32x4_t qf[QP], kf[QP];
+#pragma unroll
+    for (int c = 0; c < QP; ++c) {
+      const int d0 = 8 * c + 4 * hf;
+      qf[c] = (row_ok && d0 < a.d) ? *reinterpret_cast<const u32x4_t*>(qr + d0) : zero4;
+      kf[c] = d0 < a.d ? *reinterpret_cast<const u32x4_t*>(kr + d0) : zero4;
+    }
+    // mask of keys nb + 8(r/4) + r%4
+    const int nb = nw + 4 * hf;
+    const int64_t moff = b * a.mB + h * a.mH + (int64_t)(i0 + l32) * a.mI;
+    float mv[MASK != 0 ? 16 : 1];  // MASK 1: 0 drops the key
+    if constexpr (MASK != 0) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int n = nb + 8 * (r >> 2) + (r & 3);
+        mv[r] = 0.f;
+        if (n < lim) {
+          if constexpr (MASK == 1) mv[r] = reinterpret_cast<const uint8_t*>(a.mask)[moff + n * a.mJ] != 0 ? 1.f : 0.f;
+          else mv[r] = reinterpret_cast<const float*>(a.mask)[moff + n * a.mJ];
+        }
+      }
+    }
+    f32x16_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int c = 0; c < QP; ++c) Mfma<float>::step(acc, kf[c], qf[c]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float y = acc[r] * a.scale;
+      if constexpr (MASK == 1) y = mv[r] != 0.f ? y : -INFINITY;
+      if constexpr (MASK == 2) y += mv[r];
+      s[r] = nb + 8 * (r >> 2) + (r & 3) < lim ? y : -INFINITY;
+      bm = fmaxf(bm, s[r]);
+    }
+    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+  }
+  if (hf == 0) block_max[w][l32] = bm;
+  __syncthreads();
+  float m[CB + 1];  // the maximum before block j
+  m[0] = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < CB; ++j) m[j + 1] = fmaxf(m[j], block_max[j][l32]);
+  auto base = [&](int j) { return m[j + 1] == -INFINITY ? 0.f : m[j + 1]; };
+  if (nw < kend) {
+    float own = base(0);
+#pragma unroll
+    for (int j = 1; j < CB; ++j) own = w == j ? base(j) : own;
+    float part = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = f32_exp(s[r], own);
+      ps[w][r][lane] = p;
+      part += p;
+    }
+    parts[w][lane] = part;
+  }
+  __syncthreads();
+  float l = 0.f;
+  f32x16_t o;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) o[r] = 0.f;
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    if (n0 + 32 * j >= kend) break;
+    {
+#pragma clang fp contract(off)  // the sum is rounded after the rescale, as in f32_attn_kernel
+      const float cc = m[j + 1] > m[j] ? f32_exp(m[j], base(j)) : 1.f;
+      l = l * cc;
+      l = l + parts[j][lane];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] *= cc;
+    }
+    if (w < OF) {
+      float p[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = ps[j][r][lane];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float x = n0 + 32 * j + 8 * (r >> 2) + 4 * hf + (r & 3) < a.lk ? xv[j][r] : 0.f;
+        o = __builtin_amdgcn_mfma_f32_32x32x2f32(x, p[r], o, 0, 0, 0);
+      }
+    }
+  }
+  const float lc = l + __shfl_xor(l, 32, 64);
+  if (!row_ok) return;
+  const int64_t row = pair * a.lq + i0 + l32;
+  float* const dst = a.chunks > 1 ? a.partial + ((int64_t)chunk * a.pairs * a.lq + row) * a.dv : a.out + row * a.dv;
+  if (a.chunks > 1 && w == 0 && hf == 0)
+    *reinterpret_cast<f32x2_t*>(a.stats + 2 * ((int64_t)chunk * a.pairs * a.lq + row)) = f32x2_t{m[CB], lc};
+  if (w < OF) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int col = 32 * w + 8 * j + 4 * hf;
+      const f32x4_t x = {o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+      if (col < a.dv) *reinterpret_cast<f32x4_t*>(dst + col) = a.chunks > 1 ? x : f32_final(x, m[CB], lc);
+    }
+  }
+}
+
 // The chunks of a split launch, four output elements per thread.
 __global__ __launch_bounds__(256) void f32_combine_kernel(F32AttnArgs a) {
   const int64_t n = a.pairs * a.lq * (a.dv / 4);
@@ -421,10 +573,32 @@ static int launch_f32_masks(F32AttnArgs a, int mask_kind, hipStream_t s) {
   }
   return BIOPS_OK;
 }
+template <int QP, int OF>
+static int launch_f32_few(F32AttnArgs a, int mask_kind, hipStream_t s) {
+  if (a.chunks == 0) a.chunks = 1;
+  const dim3 grid((unsigned)(a.pairs * cdiv(a.lq, 32) * a.chunks)), block(256);
+  if (mask_kind == 0) hipLaunchKernelGGL((f32_few_kernel<QP, OF, 0>), grid, block, 0, s, a);
+  else if (mask_kind == 1) hipLaunchKernelGGL((f32_few_kernel<QP, OF, 1>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((f32_few_kernel<QP, OF, 2>), grid, block, 0, s, a);
+  return check_launch("f32_few_kernel");
+}
+// Up to two workgroups of 32 rows and 128 keys per compute unit (more of them read K and V too often:
+// 16 x 16 heads x 128 x 128, head size 64, 1024 workgroups, 17.6 -> 32.3 us), and not for a single block of
+// keys with head sizes up to 96, which has nothing to spread (8 heads x 32 x 32, head size 64, 6.9 against
+// 8.1 us).  MI355X, f32_attn_kernel against this, and with scores in memory: 8 heads x 100 x 100, head size
+// 128, 26.7 -> 14.9 us (18.9); 200 x 200 28.0 -> 18.5 (22.7); 1 x 256 25.1 -> 16.2 (16.2); 1 head x 65 x 600
+// 27.3 -> 18.9 (38.1); 8 heads x 16 x 2048 31.6 -> 23.0 (69.8); 8 x 65 x 65, head size 64, 12.7 -> 10.2 (17.5).
+template <int DP>
+static bool f32_few(const F32AttnArgs& a) {
+  const int64_t chunks = a.partial ? a.chunks : 1;
+  return (a.partial || a.lk <= kF32Chunk) && (DP > 96 || a.lk > kF32Keys) &&
+         a.pairs * cdiv(a.lq, 32) * chunks <= 2 * (int64_t)device_cus();
+}
 template <int DP, int QP, int DVP>
 static int launch_f32_attn(const F32AttnArgs& a, int mask_kind, hipStream_t s) {
-  if (!a.partial) return launch_f32_masks<DP, QP, DVP, false>(a, mask_kind, s);
-  const int rc = launch_f32_masks<DP, QP, DVP, true>(a, mask_kind, s);
+  const bool few = f32_few<DP>(a);
+  if (!a.partial) return few ? launch_f32_few<QP, DVP / 32>(a, mask_kind, s) : launch_f32_masks<DP, QP, DVP, false>(a, mask_kind, s);
+  const int rc = few ? launch_f32_few<QP, DVP / 32>(a, mask_kind, s) : launch_f32_masks<DP, QP, DVP, true>(a, mask_kind, s);
   if (rc != BIOPS_OK) return rc;
   hipLaunchKernelGGL(f32_combine_kernel, dim3((unsigned)cdiv(a.pairs * a.lq * (a.dv / 4), 256)), dim3(256), 0, s, a);
   return check_launch("f32_combine_kernel");

@@ -235,3 +235,35 @@ def test_f32_sdpa_values_behind_a_mask(B, monkeypatch):
     assert int(out.isnan().sum()) == 3 * B * 400
     monkeypatch.setenv("BIOPS_ATTENTION_MATERIALIZE", "1")
     assert torch.equal(sdpa(q, k, v, attn_mask=mask).isnan(), out.isnan())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ("full", "causal", "boolean", "additive"))
+@pytest.mark.parametrize("D,Dv", ((4, 64), (64, 8), (72, 72), (80, 40), (96, 96), (100, 128), (128, 36)))
+@pytest.mark.parametrize("lq,lk", ((1, 1), (31, 33), (33, 128), (65, 129), (40, 260)))
+def test_f32_sdpa_of_few_rows_has_the_bits_of_a_large_launch(lq, lk, D, Dv, kind):
+    """One sample (a workgroup per 32 query rows and 128 keys) and a batch that fills the chip."""
+    B, H = 160, 8
+    seed = 9860 + lk
+    q, k, v = randn(B, H, lq, D, seed=seed).cuda(), randn(B, 2, lk, D, seed=seed + 1).cuda(), randn(B, 2, lk, Dv, seed=seed + 2).cuda()
+    k *= torch.linspace(0.5, 4, lk, device="cuda").view(-1, 1)  # the maximum grows from block to block
+    v[7, 0, 0, 0] = math.inf
+    mask = None
+    if kind in ("boolean", "additive"):
+        g = torch.Generator().manual_seed(seed + 3)
+        mask = torch.rand(B, 1, lq, lk, generator=g) > 0.3
+        mask[:, :, ::3, :32] = False  # a block, and for some rows more, without a visible key
+        mask[:, :, 1::5, :128] = False
+        if kind == "additive":
+            mask = torch.where(mask, torch.rand(B, 1, lq, lk, generator=g) * -5, torch.tensor(-math.inf))
+        mask = mask.cuda()
+
+    def run(rows):
+        return sdpa(q[rows], k[rows], v[rows], attn_mask=None if mask is None else mask[rows],
+                    is_causal=kind == "causal", enable_gqa=True)
+
+    full = run(slice(None))
+    for j in (0, 7, B - 1):
+        one = slice(j, j + 1)
+        assert torch.equal(run(one).isnan(), full[one].isnan())
+        assert_bitwise(run(one).nan_to_num(1.0), full[one].nan_to_num(1.0), f"sample {j}")
