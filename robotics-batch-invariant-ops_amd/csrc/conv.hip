@@ -302,6 +302,19 @@ static unsigned elementwise_grid(int64_t total) {
 
 using namespace biops;
 
+// conv_im2col_kernel counts rows, columns of a row and wavefront units in 32 bits (room for one more
+// step and grid stride).  A patch or weight row is at least 128 bytes, so what it refuses needs
+// 512 GiB of rows, or rows of 8 GiB.
+static bool im2col_fits(const ConvShape& c, int elt) {
+  const int64_t lim = (int64_t(1) << 32) - (int64_t(1) << 19);
+  const int64_t rows = c.B * c.G * c.Lout, quads = c.Kp / (4 * (16 / elt));
+  if (rows >= lim || c.Cout >= lim || c.Kp >= lim || cdiv(c.Cout, 16) + cdiv(rows, 16) >= lim / std::max<int64_t>(quads, 1))
+    return false;
+  for (int i = 0; i < 3; ++i)
+    if (c.k[i] >= (int64_t(1) << 31)) return false;
+  return true;
+}
+
 extern "C" int64_t biops_conv_workspace_size(int dtype, int nd, int transposed, int64_t batch, int64_t cin,
                                              const int64_t* in_size, int64_t cout, const int64_t* ksize,
                                              const int64_t* stride, const int64_t* padding,
@@ -310,6 +323,10 @@ extern "C" int64_t biops_conv_workspace_size(int dtype, int nd, int transposed, 
   if (conv_shape(dtype, nd, transposed, batch, cin, in_size, cout, ksize, stride, padding, dilation, groups, c) !=
       BIOPS_OK)
     return -1;
+  if (!c.transposed && !c.depthwise1d && !im2col_fits(c, dtype_bytes(dtype))) {
+    set_error("convolution too large");
+    return -1;
+  }
   return conv_workspace(c, dtype_bytes(dtype)).total;
 }
 
@@ -349,10 +366,7 @@ extern "C" int biops_conv(int dtype, int nd, int transposed, int64_t batch, int6
       return fail(BIOPS_ERR_SIZE, "spatial extent too large");
 
   if (!c.transposed) {
-    // 32-bit rows and units (a patch row is at least 128 bytes: more would not fit the memory)
-    if (c.Cout >= (int64_t(1) << 31) || c.B * c.G >= (int64_t(1) << 31) || c.Kp >= (int64_t(1) << 31) ||
-        c.B * c.G * c.Lout >= (int64_t(1) << 31) || ws.total / 64 >= (int64_t(1) << 32))
-      return fail(BIOPS_ERR_SIZE, "convolution too large");
+    if (!im2col_fits(c, elt)) return fail(BIOPS_ERR_SIZE, "convolution too large");
     // weights [C_out, Kc] -> [C_out, Kp], unless they are whole GEMM steps already
     const bool in_place = c.Kc == c.Kp && reinterpret_cast<uintptr_t>(w) % 16 == 0;
     Im2colArgs ia{};

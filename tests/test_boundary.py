@@ -95,6 +95,25 @@ def test_conv_argument_rules_need_no_gpu():
     assert L.biops_conv_workspace_size(2, 2, 0, 2, 4, ptrs[0], 6, ptrs[1], ptrs[2], ptrs[3], ptrs[4], 3) == -1
 
 
+def test_convolutions_are_taken_up_to_the_memory():
+    """Patch rows are counted in 32 bits: 2^31 rows of 128 bytes (256 GiB) are taken, twice that is not."""
+    import ctypes
+    L = lib()
+    arr = lambda *v: (ctypes.c_int64 * len(v))(*v)  # noqa: E731
+
+    def size(batch, side, cin=1, cout=1, k=1):
+        sizes = [arr(side, side), arr(k, k), arr(1, 1), arr(0, 0), arr(1, 1)]
+        ptrs = [ctypes.addressof(a) for a in sizes]
+        return L.biops_conv_workspace_size(2, 2, 0, batch, cin, ptrs[0], cout, ptrs[1], ptrs[2], ptrs[3], ptrs[4], 1)
+
+    rows = 1 << 31
+    assert size(rows >> 20, 1 << 10) == 256 + rows * 128
+    assert size(rows >> 19, 1 << 10) == -1
+    # columns of a row: channels x taps
+    assert size(1, 2, cin=1 << 31) == (1 << 31) * 2 + 4 * (1 << 31) * 2
+    assert size(1, 2, cin=1 << 32) == -1 and size(1, 1, cin=64, cout=1 << 32) == -1
+
+
 def test_fast_call_module_matches_the_ctypes_binding():
     """The CPython fast-call module (built beside libbiops.so) reaches the same entry points
     with the same arguments: the host checks give the same status codes; wrong argument counts
