@@ -398,7 +398,7 @@ def _softmax_impl(input, dim, out_dtype, is_log):
 
 
 def softmax(input: torch.Tensor, dim: int = -1, *, dtype: torch.dtype | None = None) -> torch.Tensor:
-    """Batch-invariant softmax along any dimension (one wavefront per row, fixed tree).
+    """Batch-invariant softmax along any dimension (one wavefront or workgroup per row, fixed tree).
 
     Reference: softmax/_softmax_kernel (batch_invariant_ops.py:1074-1145).  An all -inf row
     gives 0 (not NaN); ``dtype`` sets the output dtype.

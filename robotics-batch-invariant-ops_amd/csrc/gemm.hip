@@ -366,8 +366,8 @@ static bool cfg_ok(int dtype, int c, bool swiglu, bool grouped) {
 // save whole rounds, which the 16-bit rates below cannot express.  Per-K and fixed times fitted
 // on MI355X to 40 shapes (M 16-2048, K 64-4096, N 64-4096, batches to 128, both B layouts) with every
 // entry forced: the choice is within 1 % of the best entry on geometric average and within 12 %
-// everywhere; the 16-bit model was 7 % off (16 x 1024 x 576 x 576 152.9 -> 112 us, 1020 x 3936 x
-// 1044 162 -> 134, 408 x 768 x 4096 34.3 -> 31.1).
+// everywhere; the 16-bit model was 7 % off (M x N x K: 16 x 1024 x 576 x 576 152.9 -> 112 us, 1020 x 1044 x
+// 3936 162 -> 134, 408 x 4096 x 768 34.3 -> 31.1).
 static const int kF32Slots[kNumCfg] = {0, 1, 2, 1, 2, 2, 4, 0, 1, 0, 1, 1};
 static const double kF32PerK[kNumCfg] = {0, .115, .127, .033, .033, .0188, .0202, 0, .060, 0, .114, .1135};
 static const double kF32PerKAlone[kNumCfg] = {0, 0, .064, 0, .0183, 0, 0, 0, 0, 0, 0, 0};
@@ -517,7 +517,8 @@ static int pick_cfg(int dtype, const BmmArgs& a, int epi, bool direct, bool skin
   // of 32 or 64 columns in one round with 2 to 8 of them down M (512 x 2048 x 8192 38.4 ->
   // 33.0 us, 300 x 3000 x 2048 11.7 -> 10.3 us, 128 x 8192 x 2048 12.7 -> 12.2 us; 16 down M
   // lost: 1024 x 1024 x 4096 19.0 -> 19.8 us).
-  // fp32 takes it from K = 448 on (below that it was even with the table entries or lost: 58 x 96 x 472 7.7 against 6.4 us, 475 x 224 x 608 10.0 against 9.0).
+  // fp32 takes it from K = 448 on (below that it was even with the table entries or lost: 58 x 472 x 96
+  // 7.7 against 6.4 us, 475 x 608 x 224 10.0 against 9.0).  Shapes are M x N x K.
   const int64_t row_blocks = batch * cdiv(a.M, 32), row_blocks64 = batch * cdiv(a.M, 64);
   if (skinny_ok && (dtype != BIOPS_F32 || a.K >= 448) && (row_blocks * cdiv(a.N, 32) <= cus ||
                     (row_blocks >= 2 && a.K >= 1024 && row_blocks * cdiv(a.N, 64) <= cus) ||

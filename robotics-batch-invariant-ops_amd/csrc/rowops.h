@@ -253,8 +253,8 @@ __device__ __forceinline__ void attn_softmax_row(T* row, int64_t cols, const Att
 
 // Softmax / log-softmax of R rows (row r at in + r*ld_in) by one wavefront when a row has at
 // most 64*NC chunks (NC <= kRowRegChunks): the loads of all R rows are issued before the first
-// reduction, so a wavefront keeps R*NC chunks per lane in flight.  Per row, the arithmetic and
-// reduction order are those of softmax_row.  Rows r >= nrows are skipped.
+// reduction, so a wavefront keeps R*NC chunks per lane in flight.  Per row, the reduction tree is
+// the one above.  Rows r >= nrows are skipped.
 template <typename Tin, typename Tout, int MODE, int R, int NC>
 __device__ __forceinline__ void softmax_rows_fit(const Tin* in, int64_t ld_in, Tout* out, int64_t ld_out,
                                                  int nrows, int64_t cols) {

@@ -44,7 +44,7 @@ __device__ __forceinline__ float block_max(float v, float* part) {
 // write; one wavefront per row, as the shorter rows have, leaves most of the chip idle at the row
 // counts of a decoding batch.  The same rule for every row count: the tree may depend on the row
 // length only.  MI355X, one wavefront per row with element-wise loads of misaligned rows ->
-// this: log-softmax [32, 50257] fp32 217 -> 13.2 us, softmax [64, 32000] bf16 57 -> 8.5 us,
+// this: log-softmax [32, 50257] fp32 217 -> 12.5 us a call, softmax [64, 32000] bf16 57 -> 6.4 us,
 // [4096, 8192] bf16 44.3 -> 22.8 us (5.9 TB/s of read + write), [1, 131072] fp32 376 -> 38 us.
 template <typename Tin, typename Tout, int MODE, int T, int NC, bool LOOP>
 __global__ __launch_bounds__(T) void softmax_block_kernel(SoftmaxArgs a) {
