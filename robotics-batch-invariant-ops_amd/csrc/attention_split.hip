@@ -47,7 +47,8 @@ constexpr int kSplitKeys = 256;      // keys per workgroup of split_score_kernel
 //   fill the chip: 1 row 337 -> 61 us (8 heads per kv head), 16 rows 172 -> 121 (4 heads), 340 ->
 //   165 (8 heads); more rows were not measured on this form;
 //   keys, 1 sample, 4 heads, one row: 700 keys 32.5 -> 12.2.  A second launch costs about 2 us of
-//   host time, so calls up to 512 keys, which the host bounds either way, stay on the fused kernel.
+//   host time, so calls up to 512 keys, which the host bounds either way, stay on the fused kernel
+//   (replayed from a graph, without that cost, 400 keys would gain too).
 constexpr int kSplitMaxQuery = 16;   // query rows per head
 constexpr int kSplitMinKeys = 512;   // longer key ranges are split
 // The fused kernel needs no workspace, so this path must not make a call run out of memory that

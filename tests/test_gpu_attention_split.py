@@ -159,6 +159,34 @@ def test_query_rows_in_chunks_give_the_bits_of_one_call(dtype, mask_kind, shape)
             assert_bitwise(part, whole[:, :, rows], f"rows from {first}")
 
 
+# Row and column blocks of the value kernel by launch size (256 compute units): (batch, query heads, kv
+# heads, query rows, keys, head size, value size), blocks of rows x columns.
+LAUNCHES = (
+    ((100, 8, 2, 2, 530, 64, 64), "16 x 64"),
+    ((150, 8, 2, 1, 530, 64, 72), "16 x 128"),
+    ((40, 8, 2, 1, 2500, 64, 64), "4 x 32"),
+    ((60, 8, 2, 1, 2500, 64, 128), "4 x 64"),
+    ((100, 8, 2, 1, 2500, 64, 128), "4 x 128"),
+    ((15, 16, 2, 1, 2100, 64, 128), "8 x 16"),
+    ((30, 16, 2, 1, 2100, 64, 128), "8 x 32"),
+    ((60, 16, 2, 1, 2100, 64, 128), "8 x 64"),
+    ((80, 16, 2, 1, 2100, 64, 128), "8 x 128"),
+    ((64, 14, 2, 4, 600, 64, 136), "32 x 64"),
+    ((64, 14, 2, 6, 600, 64, 136), "64 x 128"),
+)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,blocks", LAUNCHES)
+def test_value_blocks_give_the_bits_of_one_call(shape, blocks):
+    B, Hq, Hkv, Lq, Lk, D, Dv = shape
+    g = torch.Generator("cuda").manual_seed(9470)
+    q, k, v = (torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+               for s in ((B, Hq, 20, D), (B, Hkv, Lk, D), (B, Hkv, Lk, Dv)))
+    whole = sdpa(q, k, v, enable_gqa=True)
+    assert_bitwise(sdpa(q[:, :, :Lq], k, v, enable_gqa=True), whole[:, :, :Lq], blocks)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DTYPES16)
 def test_infinities_and_nan_in_chunks_of_query_rows(dtype):
