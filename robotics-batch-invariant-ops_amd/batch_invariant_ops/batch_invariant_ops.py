@@ -609,11 +609,13 @@ def _f32_attention_ok(B, Hq, Lq, Lk, D, Dv):
 
 def _f32_rows(t):
     """``t`` [B, H, L, D] with the 16-byte aligned rows that the one-pass float32 kernel reads, copied
-    where a view has others, and its strides (0 for dimensions of one element)."""
+    where a view has others (dimensions it repeats stay repeated), and its strides (0 for dimensions
+    of one element)."""
     strides = [st if n > 1 else 0 for n, st in zip(t.shape[:-1], t.stride())]
     if t.data_ptr() % 16 or strides[2] >= 1 << 25 or any(st % 4 for st in strides):
-        t = t.clone(memory_format=torch.contiguous_format)
-        strides = t.stride()[:-1]
+        once = t[tuple(slice(0, 1) if st == 0 else slice(None) for st in strides)]
+        t = once.clone(memory_format=torch.contiguous_format).expand(t.shape)
+        strides = [st if n > 1 else 0 for n, st in zip(t.shape[:-1], t.stride())]
     return t, strides
 
 

@@ -179,7 +179,7 @@ def test_f32_sdpa_probabilities_to_the_last_bits():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("layout", ("base", "pitch", "keys", "wide"))
+@pytest.mark.parametrize("layout", ("base", "pitch", "keys", "wide", "shared"))
 def test_f32_sdpa_views_give_the_bits_of_their_copies(layout):
     """Rows that are not 16-byte aligned (an offset base, an odd pitch, keys behind an odd offset) and
     rows further apart than the kernel's 32-bit offsets take the same path as an aligned copy."""
@@ -190,6 +190,8 @@ def test_f32_sdpa_views_give_the_bits_of_their_copies(layout):
             return randn(B * H * L * D + 1, seed=seed).cuda()[1:].view(B, H, L, D)
         if layout == "pitch":
             return randn(B, L, H, D + 1, seed=seed).cuda()[..., :D].transpose(1, 2)
+        if layout == "shared":  # one odd-pitch sample and head for all
+            return randn(1, 1, L, D + 1, seed=seed).cuda()[..., :D].expand(B, H, L, D)
         if layout == "keys":
             return randn(B, H, L * D + 3, seed=seed).cuda()[..., 3:].view(B, H, L, D)
         t = torch.empty(((L - 1) << 25) + D, device="cuda").as_strided((1, 1, L, D), (0, 0, 1 << 25, 1))
@@ -267,3 +269,15 @@ def test_f32_sdpa_of_few_rows_has_the_bits_of_a_large_launch(lq, lk, D, Dv, kind
         one = slice(j, j + 1)
         assert torch.equal(run(one).isnan(), full[one].isnan())
         assert_bitwise(run(one).nan_to_num(1.0), full[one].nan_to_num(1.0), f"sample {j}")
+
+
+@pytest.mark.gpu
+def test_f32_rows_keep_what_a_view_repeats():
+    """The aligned copy of an operand that is repeated over samples, heads or rows has it once."""
+    from batch_invariant_ops.batch_invariant_ops import _f32_rows
+
+    t = torch.arange(7 * 5, dtype=torch.float32, device="cuda").view(1, 1, 7, 5)[..., :4]
+    for view in (t.expand(3, 2, 7, 4), t[:, :, 2:3].expand(3, 2, 6, 4), t[:, :, :1], t[:, :, :0].expand(3, 2, 0, 4)):
+        rows, strides = _f32_rows(view)
+        assert torch.equal(rows, view) and rows.data_ptr() % 16 == 0 and all(st % 4 == 0 for st in strides)
+        assert rows.untyped_storage().nbytes() <= 7 * 5 * 4
